@@ -24,7 +24,10 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 LIB_NAME = "libfa_mi355x.so"
 EXT_NAME = "fa_p100_ext"
-KERNEL_SOURCES = ["fa_fwd.hip", "fa_bwd.hip", "fa_mask.hip", "fa_capi.hip"]
+KERNEL_SOURCES = ["fa_launch.hip", "fa_mask.hip", "fa_capi.hip"]
+# Compiled once per tile width and format (-DFA_WIDTH, -DFA_BF), the slowest first.
+WIDTH_SOURCES = ["fa_bwd.hip", "fa_fwd.hip"]
+WIDTHS = [128, 96, 64, 256, 32]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -67,10 +70,13 @@ def build_kernels(jobs=8):
     hipcc = os.path.join(ROCM, "bin", "hipcc")
     objs = []
     cmds = []
-    for src in KERNEL_SOURCES:
-        obj = os.path.join(OBJ, src.replace(".hip", ".o"))
+    units = [(src, (w, bf)) for src in WIDTH_SOURCES for w in WIDTHS for bf in (0, 1)]
+    for src, unit in units + [(src, None) for src in KERNEL_SOURCES]:
+        name = src.replace(".hip", "_{}_{}.o".format(*unit) if unit else ".o")
+        obj = os.path.join(OBJ, name)
         objs.append(obj)
-        cmds.append([hipcc, *HIPCC_FLAGS, *FILE_FLAGS.get(src, []), "-c",
+        define = ["-DFA_WIDTH={}".format(unit[0]), "-DFA_BF={}".format(unit[1])] if unit else []
+        cmds.append([hipcc, *HIPCC_FLAGS, *FILE_FLAGS.get(src, []), *define, "-c",
                      os.path.join(CSRC, src), "-o", obj])
     with ThreadPoolExecutor(max_workers=min(jobs, len(cmds))) as ex:
         list(ex.map(_run, cmds))

@@ -70,16 +70,15 @@ static_assert(kTile == kBwdTile, "workspace layout assumes this key tile");
 // registers per lane at one wave per SIMD), the streamed tiles have 32 rows
 // and the K operands come straight from global memory into registers (a
 // resident K tile would not fit in LDS beside V and the staged tiles).
-// W4 (width 64, grids of at least two workgroups per CU): one wave per row
+// W4 (width 64, where bwd_plan takes it): one wave per row
 // block and 32-row streamed tiles as at width 256, but K resident in LDS and
 // at most 256 registers per wave (the kernel needs ~170), so two workgroups
 // (54 KB of LDS each) share a CU on separate barriers and one's softmax runs
 // beside the other's products. Same-box A/B, bwd_main at H=16 N=4096 D=64
 // causal: -4% (minimum) and -7% (median of five rounds); within 0.6% at
 // H=16 N=4096 D=64 dense and at H=16/8 N=8192 D=64 causal; +17% at H=16
-// N=2048 D=64 causal, whose 256 workgroups leave one per CU, so the launcher
-// takes it only where the grid fills both slots. (At width 128 two such
-// workgroups do not fit in LDS.)
+// N=2048 D=64 causal, whose 256 workgroups leave one per CU, which bwd_plan's
+// estimate weighs. (At width 128 two such workgroups do not fit in LDS.)
 template <int D, bool W4 = false>
 struct BwdShape {
   static constexpr int kWaves = D > 128 || W4 ? 4 : 8;
@@ -107,8 +106,9 @@ constexpr int kSplitBias = 5;
 // causal (two boxes): 100 beat 86 by 1.4%, 115 and 130 lost; at H=16/8
 // N=8192 D=64 within 0.7%.
 constexpr int kSplitNumW4 = 100;
-// The FEAT bit that selects W4 (kept clear of the per-score input bits).
-constexpr int kBwdW4 = 16;
+// The FEAT bits that select W4 and the instantiations whose work items are the
+// phases apart (BwdPlan::apart), kept clear of the per-score input bits.
+constexpr int kBwdW4 = 16, kBwdApart = 32;
 
 // LDS: every tile is its own __shared__ object (declared in bwd_kernel), so
 // the compiler can tell that a step's reads never touch the tiles that the
@@ -172,9 +172,10 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(const half_t* __restrict__
 }
 
 // Direct load of 64 consecutive floats (rows r0 .. r0+63 of a per-row
-// vector; rows past its end read as zeros).
-__device__ __forceinline__ void vec_load64(float* lds, rsrc_t r, int r0, int lane) {
-  lds_direct_buf<4>(lds, r, (uint32_t)lane * 4u, (uint32_t)r0 * 4u);
+// vector; rows past its end read as zeros) to byte_off of an LDS run.
+__device__ __forceinline__ void vec_load64(float* lds, rsrc_t r, int r0, int lane,
+                                           uint32_t byte_off) {
+  lds_direct_buf<4>(lds, r, (uint32_t)lane * 4u, (uint32_t)r0 * 4u, byte_off);
 }
 
 // Exchange of per-wave accumulators: waves of the upper half (w >= 4) store
@@ -213,7 +214,7 @@ __device__ __forceinline__ void partial_add(const float* region, floatx16 (&acc)
 // non-coherent copies). Slot layout [w4][k][g4][lane] x 4 floats: every
 // instruction moves 1 KB of consecutive bytes.
 constexpr int kDeviceCoherent = 16;  // sc1 bit of the buffer intrinsics' cache-policy operand
-template <int n>
+template <int n, int POLICY = kDeviceCoherent>
 __device__ __forceinline__ void slot_store(rsrc_t r, const floatx16 (&acc)[n], int w4, int lane) {
 #pragma unroll
   for (int k = 0; k < n; ++k)
@@ -221,7 +222,7 @@ __device__ __forceinline__ void slot_store(rsrc_t r, const floatx16 (&acc)[n], i
     for (int g4 = 0; g4 < 4; ++g4) {
       const floatx4 v = {acc[k][4 * g4], acc[k][4 * g4 + 1], acc[k][4 * g4 + 2], acc[k][4 * g4 + 3]};
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, lane * 16,
-                                             ((w4 * n + k) * 4 + g4) * 1024, kDeviceCoherent);
+                                             ((w4 * n + k) * 4 + g4) * 1024, POLICY);
     }
 }
 template <int n>
@@ -429,7 +430,8 @@ struct QWave {
                       (mwh & 0x0F0F0F0Fu) == 0x0F0F0F0Fu;
     const bool edge = SPLIT    ? __builtin_amdgcn_ballot_w64(!open) != 0
                       : BOUNDS ? true
-                               : CAUSAL && __builtin_amdgcn_ballot_w64(lo < 27) != 0;
+                      : CAUSAL ? __builtin_amdgcn_ballot_w64(lo < 27) != 0
+                               : __builtin_amdgcn_ballot_w64(hi < 28) != 0;
     auto softmax = [&](auto edge_tag) {
       constexpr bool EDGE = decltype(edge_tag)::value;
 #pragma unroll
@@ -437,6 +439,7 @@ struct QWave {
         const int idx = 8 * (r >> 2) + (r & 3);
         float p = fast_exp2(fmaf(st[r], c, -lse2));
         if (CAUSAL && EDGE) p = (idx <= lo) ? p : 0.f;
+        if (!BOUNDS && !CAUSAL && EDGE) p = (idx < hi) ? p : 0.f;
         if (BOUNDS && EDGE) p = (idx < hi && idx >= lw && ((mwh >> idx) & 1u)) ? p : 0.f;
         // Dropout: the gradient of P is the kept dP scaled by zs.
         const bool keep = (zwh >> idx) & 1u;
@@ -491,9 +494,10 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
     const uint32_t* __restrict__ mask_t, int mask_heads, const uint32_t* __restrict__ drop,
     const uint32_t* __restrict__ drop_t, float drop_scale, const float* __restrict__ bias,
     long long bias_sb, long long bias_sh, float bias_raw, float* __restrict__ dbias, int dr,
-    int NK, const int* __restrict__ block_rows, const int* __restrict__ block_cols) {
+    int NK, const int* __restrict__ block_rows, const int* __restrict__ block_cols, int parts) {
   constexpr bool W4 = (FEAT & kBwdW4) != 0;
-  constexpr int FI = FEAT & ~kBwdW4;  // the per-score inputs
+  constexpr bool APART = (FEAT & kBwdApart) != 0;
+  constexpr int FI = FEAT & ~(kBwdW4 | kBwdApart);  // the per-score inputs
   using Sh = BwdShape<D, W4>;
   using L = BwdLds<D, W4>;
   constexpr int kWaves = Sh::kWaves, kHalves = Sh::kHalves;
@@ -519,19 +523,54 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
   const int h = lane >> 5;
   const int l32 = lane & 31;
 
-  const int wi = xcd_work_index(n_tiles * BHkv);
-  if (wi < 0) return;
-  const int bkv = wi / n_tiles;  // over B*Hkv
+  const int n_ktiles = (NK + kTile - 1) / kTile, n_qtiles = (N + kTile - 1) / kTile;
+  // The workgroup's item: key tile tw's phase 1 and query tile tw's phase 2 of
+  // kv head bkv (over B*Hkv), the latter for query heads g_first .. g_end - 1
+  // of its group. APART: phase 1 and each query head's phase 2 are items of
+  // their own, the phase-1 items first (launch_main_t says when). Workgroups
+  // start in order, so the long items start first and the short ones fill the
+  // CUs that come free; phase 2 starts with the highest tile, whose causal
+  // item is the longest. With `parts` above one that many workgroups share a
+  // key tile's phase-1 steps, and bwd_reduce_kernel adds their sums.
+  int bkv, tw, g_first = 0, g_end = group, part = 0;
+  bool do1 = true, do2 = true;
+  if constexpr (APART) {
+    const int n1 = n_ktiles * BHkv * parts, n2 = n_qtiles * BHkv * group;
+    const int per1 = (n1 + kXcds - 1) / kXcds, per2 = (n2 + kXcds - 1) / kXcds;
+    const int xcd = blockIdx.x % kXcds, s = blockIdx.x / kXcds;
+    if (s < per1) {
+      const int w = xcd * per1 + s;
+      if (w >= n1) return;
+      const int t = w / parts;
+      part = w % parts;
+      bkv = t / n_ktiles;
+      tw = t % n_ktiles;
+      do2 = false;
+    } else {
+      const int w = xcd * per2 + s - per1;
+      if (w >= n2) return;
+      const int bh = w / n_qtiles;
+      bkv = bh / group;
+      g_first = bh % group;
+      g_end = g_first + 1;
+      tw = n_qtiles - 1 - w % n_qtiles;
+      do1 = false;
+    }
+  } else {
+    const int w = xcd_work_index(n_tiles * BHkv);
+    if (w < 0) return;
+    bkv = w / n_tiles;
+    tw = w % n_tiles;
+    do1 = tw < n_ktiles;
+    do2 = tw < n_qtiles;
+  }
   const int Hkv = Hq / group;
   const int b = bkv / Hkv, hkv = bkv % Hkv;
   // Per-entry key length (key padding), clamped to [1, NK] (NK: key rows, N:
   // query rows). kofs = NK - N: causal masking aligns the last query row with
-  // the last key row, so query i sees key j iff j <= i + kofs. Workgroup t
-  // runs phase 1 for key tile t when there is one and phase 2 for query
-  // tile t when there is one.
+  // the last key row, so query i sees key j iff j <= i + kofs.
   const int Nk = kv_len ? min(max(kv_len[b], 1), NK) : NK;
   const int kofs = NK - N;
-  const int n_ktiles = (NK + kTile - 1) / kTile, n_qtiles = (N + kTile - 1) / kTile;
   // Causal sliding window (only in the masked instantiation): row i sees keys
   // (i - Wb, i]; 0 = none.
   const int Wb = BOUNDS ? window : 0;
@@ -631,7 +670,11 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
   // on which one that is).
   // Query rows of key tile u's phase 1: from its diagonal (causal) to the end,
   // or to the last row whose window or sequence reaches the tile.
-  auto q_end = [&](int u) { return narrowed ? upper(u * kTile + kTile - 1) : N; };
+  // (No row reaches a tile wholly past the entry's key length.)
+  auto q_end = [&](int u) {
+    if (BOUNDS && u * kTile >= Nk) return 0;
+    return narrowed ? upper(u * kTile + kTile - 1) : N;
+  };
   // ... and from its diagonal (causal) or the start of its first key's
   // sequence, rounded down to a streamed tile (u * kTile is a multiple of kSub).
   auto q_start = [&](int u) {
@@ -645,14 +688,13 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
   auto split = [&](int u) {
     // (not at width 256: a second inlined copy of phase 1 spilled registers;
     // not with a block layout, whose key tiles have no common amount of work)
-    if constexpr (KG || SPARSE) return 0;
+    if constexpr (KG || SPARSE || APART) return 0;
     const int m = n_tiles - 1 - 2 * u;
     // windows leave the tiles' work equal; with kofs != 0 the key and query
     // tiles do not pair up
     if (!CAUSAL || m <= 0 || narrowed || kofs != 0) return 0;
     return max(0, min((group * m * split_num - split_bias) >> 8, n_iters(u) - 1));
   };
-  const int tw = wi % n_tiles;
   const int partner = n_tiles - 1 - tw;
   const int x_help = partner < tw ? split(partner) : 0;  // run first, for tile `partner`
   const int x_own = tw < partner ? split(tw) : 0;        // given to workgroup `partner`
@@ -669,8 +711,8 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
     const int* const clist =
         SPARSE ? block_cols + ((size_t)bkv * nb + tile) * (group * nb + 1) : nullptr;
     const int n_it = SPARSE ? clist[0] * kSpb : n_iters(tile);
-    const int it_begin = helping ? n_it - x_help : 0;
-    const int it_end = helping ? n_it : n_it - x_own;
+    const int it_begin = APART ? n_it * part / parts : helping ? n_it - x_help : 0;
+    const int it_end = APART ? n_it * (part + 1) / parts : helping ? n_it : n_it - x_own;
     const bool shared = helping || x_own > 0;
     KVWave<D, CAUSAL, BOUNDS, BF, FI == 0 || KG, kSplit> w;
     {
@@ -728,9 +770,9 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
         plan_q.part(tq, rq, i0, wave, u);
         plan_q.part(to, ro, i0, wave, u);
       }
-      if (wave == 0) vec_load64(tv, make_rsrc(Lse2 + bhq * N, (uint32_t)N * 4), i0, lane);
+      if (wave == 0) vec_load64(tv, make_rsrc(Lse2 + bhq * N, (uint32_t)N * 4), i0, lane, 0);
       if (wave == 1)
-        vec_load64(tv + kVecStride, make_rsrc(Dvec + bhq * N, (uint32_t)N * 4), i0, lane);
+        vec_load64(tv, make_rsrc(Dvec + bhq * N, (uint32_t)N * 4), i0, lane, kVecStride * 4);
     };
     // Bias values of step `it` for this lane's key and its 16 query rows,
     // through a resource over the wave's 32 rows (rows past N read zeros, a
@@ -811,6 +853,16 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
       }
     }
     bool finish = true;
+    if constexpr (APART) {
+      if (parts > 1) {  // a partial sum, for bwd_reduce_kernel
+        if (!half)
+          slot_store<2 * (D / 32), 0>(
+              make_rsrc(slots + ((size_t)(bkv * n_ktiles + tile) * parts + part) * kSlotFloats,
+                        kSlotFloats * 4),
+              w.acc, w4, lane);
+        return;
+      }
+    }
     if (shared) {
       const int u = helping ? partner : tw;
       unsigned* cnt = counters + (size_t)bkv * pairs + u;
@@ -864,7 +916,7 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
       }
     }
     // dK (scaled) and dV leave as fp16.
-    if (finish && !half && (!BOUNDS || j_col < NK)) {
+    if (finish && !half && j_col < NK) {
       half_t* dkrow = dK + kv_off + (size_t)j_col * stk.n;
       half_t* dvrow = dV + kv_off + (size_t)j_col * stk.n;
 #pragma unroll
@@ -886,17 +938,19 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
     }
     __syncthreads();  // the exchange regions are the next item's or phase's staging memory
   };
-  if (tw < n_ktiles) {
-    if (x_help > 0) run_item(true);
+  if (do1) {
+    if constexpr (!APART) {
+      if (x_help > 0) run_item(true);
+    }
     run_item(false);
   }
   const int t0 = tw * kTile;  // query rows of phase 2
 
   // ============================== phase 2: dQ ==============================
-  if (tw < n_qtiles) {
+  if (do2) {
     const int iw = t0 + w4 * 32;  // this wave's query rows
     const int i_row = iw + l32;
-    const bool row_ok = !BOUNDS || i_row < N;
+    const bool row_ok = i_row < N;
     const int kv_end = CAUSAL ? min(Nk, t0 + kTile + kofs) : row_hi(t0 + kTile - 1);
     const int lane_hi = row_hi(i_row);  // this lane's row: keys from lane_hi on are masked
     // (at least one step: rows above the first key, when there are more query
@@ -907,7 +961,7 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
     const int t_lo = narrowed ? lower(t0) / kSub : 0;
     const int key_lo = narrowed ? lower(i_row) : -(1 << 30);
 
-    for (int g = 0; g < group; ++g) {
+    for (int g = g_first; g < g_end; ++g) {
       const int hq = hkv * group + g;
       const size_t bhq = (size_t)b * Hq + hq;
       // Block-sparse: the key blocks this query block attends (count first);
@@ -1050,6 +1104,35 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
   }
 }
 
+// Sums the partial dK^T/dV^T of a key tile whose phase 1 was shared by `parts`
+// workgroups, in the order of the parts, and writes dK and dV. One float4 of a
+// slot (slot_store's layout) per thread.
+template <int D>
+constexpr int kReduceBlocks = kTile * D * 2 / 4 / 256;  // workgroups per key tile
+template <int D, bool BF>
+__global__ __launch_bounds__(256) void bwd_reduce_kernel(
+    const float* __restrict__ slots, half_t* __restrict__ dK, half_t* __restrict__ dV, int NK,
+    int Hkv, int n_ktiles, int parts, float scale, float zs, Strides stk, int dr) {
+  constexpr int kSlotFloats = kTile * D * 2;
+  const int item = blockIdx.x / kReduceBlocks<D>;  // (b * Hkv + hkv) * n_ktiles + tile
+  const int f = blockIdx.x % kReduceBlocks<D> * 256 + threadIdx.x;  // float4 of the slot
+  const float* src = slots + (size_t)item * parts * kSlotFloats + 4 * f;
+  floatx4 sum = *reinterpret_cast<const floatx4*>(src);
+#pragma unroll 4
+  for (int p = 1; p < parts; ++p)
+    sum += *reinterpret_cast<const floatx4*>(src + (size_t)p * kSlotFloats);
+  const int lane = f % 64, g4 = f / 64 % 4, k = f / 256 % (2 * (D / 32)), w4 = f / 256 / (2 * (D / 32));
+  const int j = item % n_ktiles * kTile + w4 * 32 + lane % 32;
+  const bool is_k = k >= D / 32;
+  const int col = (is_k ? k - D / 32 : k) * 32 + 8 * g4 + 4 * (lane / 32);
+  if (j >= NK || col >= dr) return;
+  const int bkv = item / n_ktiles, b = bkv / Hkv, hkv = bkv % Hkv;
+  half4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = to16<BF>(sum[e] * (is_k ? scale : zs));
+  *reinterpret_cast<half4*>((is_k ? dK : dV) + b * stk.b + hkv * stk.h + (size_t)j * stk.n + col) = r;
+}
+
 template <int D, bool BF>
 hipError_t launch_pre_d(const BwdArgs& a) {
   constexpr int kRowsPerBlock = 256 / pre_lanes_per_row(D);
@@ -1062,10 +1145,14 @@ hipError_t launch_pre_d(const BwdArgs& a) {
 }
 
 template <int D, bool CAUSAL, bool BOUNDS, int FEAT, bool BF>
-hipError_t launch_main_t(const BwdArgs& a) {
+hipError_t launch_main_t(const BwdArgs& a, const BwdPlan& plan) {
   const int NK = key_rows(a.N, a.Nkv);
   const int n_tiles = (max(a.N, NK) + kTile - 1) / kTile;
-  const dim3 grid(xcd_grid(n_tiles * a.B * a.Hkv));
+  const int n_k = (NK + kTile - 1) / kTile, n_q = (a.N + kTile - 1) / kTile;
+  constexpr bool apart = (FEAT & kBwdApart) != 0;
+  const int parts = apart ? plan.parts : 1;
+  const dim3 grid(apart ? xcd_grid(n_k * a.B * a.Hkv * parts) + xcd_grid(n_q * a.B * a.Hq)
+                        : xcd_grid(n_tiles * a.B * a.Hkv));
   using Sh = BwdShape<D, (FEAT & kBwdW4) != 0>;
   // D is the tile width; a.D the head dim in memory, which sets the default
   // scale and the strides.
@@ -1076,29 +1163,55 @@ hipError_t launch_main_t(const BwdArgs& a) {
                      (half_t*)a.dq16, (half_t*)a.dk, (half_t*)a.dv, a.N, a.Hq, a.Hq / a.Hkv, n_tiles,
                      a.B * a.Hkv, scale, scale * kLog2e, make_strides(a.layout, a.Hq, a.N, a.D),
                      make_strides(a.layout, a.Hkv, NK, a.D), a.counters, a.slots,
-                     a.slots ? ((FEAT & kBwdW4) ? kSplitNumW4 : kSplitNum) * 64 / Sh::kSub : 0,
-                     a.slots ? kSplitBias : 0, a.kv_len, a.window,
+                     a.counters ? ((FEAT & kBwdW4) ? kSplitNumW4 : kSplitNum) * 64 / Sh::kSub : 0,
+                     a.counters ? kSplitBias : 0, a.kv_len, a.window,
                      a.alibi, a.seg_start, a.seg_end, a.mask, a.mask_t, a.mask_heads, a.drop,
                      a.drop_t, a.drop_scale, a.bias, a.bias_sb, a.bias_sh,
-                     a.bias ? 1.f / scale : 0.f, a.dbias, a.D, NK, a.block_rows, a.block_cols);
+                     a.bias ? 1.f / scale : 0.f, a.dbias, a.D, NK, a.block_rows, a.block_cols, parts);
+  if (parts > 1) {
+    const int n = n_k * a.B * a.Hkv * kReduceBlocks<D>;
+    hipLaunchKernelGGL((bwd_reduce_kernel<D, BF>), dim3((unsigned)n), dim3(256), 0,
+                       (hipStream_t)a.stream, a.slots, (half_t*)a.dk, (half_t*)a.dv, NK, a.Hkv, n_k,
+                       parts, scale, a.drop ? a.drop_scale : 1.f,
+                       make_strides(a.layout, a.Hkv, NK, a.D), a.D);
+  }
   return hipGetLastError();
 }
 
 template <int D, bool BF>
 hipError_t launch_main_d(const BwdArgs& a) {
   // Key lengths, windows, packed sequences and ALiBi need the masked
-  // instantiation (kTile is a multiple of every kSub); a mask, dropout or a bias
-  // one of its copies with those inputs compiled in (Feat).
-  const bool bounds = (a.N % kTile) != 0 || a.kv_len != nullptr || a.window > 0 ||
-                      a.alibi != nullptr || a.seg_start != nullptr ||
-                      key_rows(a.N, a.Nkv) != a.N;
-  auto with = [&](auto feat) {
-    constexpr int F = decltype(feat)::value;
-    return a.causal ? launch_main_t<D, true, true, F, BF>(a)
-                    : launch_main_t<D, false, true, F, BF>(a);
+  // instantiation; a mask, dropout or a bias one of its copies with those
+  // inputs compiled in (Feat). A ragged N does not: rows and keys past it load
+  // as zeros, so in phase 1 such a row adds P = 1 times dO = 0 and dS = 0, and
+  // phase 2 masks the keys past N on the last step only (causal rows never see
+  // them). B=2 H=32/8 N=3001 D=128 dense, main kernel and preprocess: 1300 ->
+  // 1061 us from the masked instantiation to the unmasked one.
+  const bool bounds = a.kv_len != nullptr || a.window > 0 || a.alibi != nullptr ||
+                      a.seg_start != nullptr || key_rows(a.N, a.Nkv) != a.N;
+  const int feat = feat_of(a.mask != nullptr, a.drop != nullptr, a.bias != nullptr,
+                           a.block_rows != nullptr);
+  // (A mask and a block layout run with one item per tile: a layout and the
+  // equal mask add a key tile's steps in one order, bit for bit, which parts of
+  // unequal lists would not.)
+  const BwdPlan plan = bwd_plan(a.B, a.Hq, a.Hkv, a.N, key_rows(a.N, a.Nkv), a.D, a.causal,
+                                D == 64 && feat == 0, a.slots != nullptr);
+  auto run = [&](auto bounds_tag, auto f) {
+    constexpr bool BOUNDS = decltype(bounds_tag)::value;
+    constexpr int F = decltype(f)::value;
+    return a.causal ? launch_main_t<D, true, BOUNDS, F, BF>(a, plan)
+                    : launch_main_t<D, false, BOUNDS, F, BF>(a, plan);
   };
-  switch (feat_of(a.mask != nullptr, a.drop != nullptr, a.bias != nullptr,
-                  a.block_rows != nullptr)) {
+  // `bt`: the masked or the unmasked instantiation of the inputs F, with the
+  // phases apart where the plan has them so.
+  auto planned = [&](auto bt, auto f) {
+    constexpr int F = decltype(f)::value;
+    return plan.apart ? run(bt, std::integral_constant<int, F | kBwdApart>{}) : run(bt, f);
+  };
+  using Masked = std::true_type;
+  using Plain = std::false_type;
+  auto with = [&](auto f) { return run(Masked{}, f); };
+  switch (feat) {
     case kFeatBlock: return with(std::integral_constant<int, kFeatBlock>{});
     case kFeatBlock | kFeatDrop:
       return with(std::integral_constant<int, kFeatBlock | kFeatDrop>{});
@@ -1107,69 +1220,34 @@ hipError_t launch_main_d(const BwdArgs& a) {
       // Keep bits need no bounds: where nothing else does, the unmasked
       // instantiations (not at width 256, where they spill).
       if constexpr (D <= 128) {
-        if (!bounds)
-          return a.causal ? launch_main_t<D, true, false, kFeatDrop, BF>(a)
-                          : launch_main_t<D, false, false, kFeatDrop, BF>(a);
+        if (!bounds) return planned(Plain{}, std::integral_constant<int, kFeatDrop>{});
       }
-      return with(std::integral_constant<int, kFeatDrop>{});
+      return planned(Masked{}, std::integral_constant<int, kFeatDrop>{});
     case kFeatMask | kFeatDrop: return with(std::integral_constant<int, kFeatMask | kFeatDrop>{});
     case kFeatBias:  // (no bias at width 256: the C ABI refuses it)
       if constexpr (D > 128) return hipErrorInvalidValue;
-      else return with(std::integral_constant<int, kFeatBias>{});
+      else return planned(Masked{}, std::integral_constant<int, kFeatBias>{});
     default: break;
   }
-  if constexpr (D == 64) {  // W4 where the grid gives every CU two workgroups (BwdShape)
-    const long long wgs =
-        (long long)((max(a.N, key_rows(a.N, a.Nkv)) + kTile - 1) / kTile) * a.B * a.Hkv;
-    if (wgs >= 2LL * kCUs) {
-      if (a.causal)
-        return bounds ? launch_main_t<D, true, true, kBwdW4, BF>(a)
-                      : launch_main_t<D, true, false, kBwdW4, BF>(a);
-      return bounds ? launch_main_t<D, false, true, kBwdW4, BF>(a)
-                    : launch_main_t<D, false, false, kBwdW4, BF>(a);
-    }
+  if constexpr (D == 64) {
+    if (plan.w4)
+      return bounds ? planned(Masked{}, std::integral_constant<int, kBwdW4>{})
+                    : planned(Plain{}, std::integral_constant<int, kBwdW4>{});
   }
-  if (a.causal)
-    return bounds ? launch_main_t<D, true, true, 0, BF>(a)
-                  : launch_main_t<D, true, false, 0, BF>(a);
-  return bounds ? launch_main_t<D, false, true, 0, BF>(a)
-                : launch_main_t<D, false, false, 0, BF>(a);
+  return bounds ? planned(Masked{}, std::integral_constant<int, 0>{})
+                : planned(Plain{}, std::integral_constant<int, 0>{});
 }
 
 }  // namespace
 
-unsigned long long bwd_launch_items(int B, int Hq, int Hkv, int N, int D, int Nkv) {
-  const unsigned long long rows = (unsigned long long)B * Hq * N;
-  const unsigned long long rows_per_block = 256 / pre_lanes_per_row(padded_head_dim(D));
-  const unsigned long long pre = (rows + rows_per_block - 1) / rows_per_block * 256;
-  const unsigned long long tiles =
-      ((unsigned long long)(N > key_rows(N, Nkv) ? N : key_rows(N, Nkv)) + kTile - 1) / kTile;
-  const unsigned long long wgs = tiles * (unsigned long long)B * (unsigned long long)Hkv;
-  const unsigned long long threads = padded_head_dim(D) > 128 ? 256 : 512;  // BwdShape
-  const unsigned long long main = (wgs + kXcds - 1) / kXcds * kXcds * threads;
-  return pre > main ? pre : main;
+// One object file per width and format (-DFA_WIDTH, -DFA_BF), compiled in parallel.
+template <>
+hipError_t launch_bwd_pre_w<FA_WIDTH, FA_BF>(const BwdArgs& a) {
+  return launch_pre_d<FA_WIDTH, FA_BF>(a);
 }
-
-hipError_t launch_bwd_preprocess(const BwdArgs& a) {
-  const int w = padded_head_dim(a.D);
-  if (a.dtype == kBF16)
-    return w == 32 ? launch_pre_d<32, true>(a) : w == 64 ? launch_pre_d<64, true>(a)
-         : w == 96 ? launch_pre_d<96, true>(a) : w == 128 ? launch_pre_d<128, true>(a)
-         : launch_pre_d<256, true>(a);
-  return w == 32 ? launch_pre_d<32, false>(a) : w == 64 ? launch_pre_d<64, false>(a)
-       : w == 96 ? launch_pre_d<96, false>(a) : w == 128 ? launch_pre_d<128, false>(a)
-       : launch_pre_d<256, false>(a);
-}
-
-hipError_t launch_bwd_main(const BwdArgs& a) {
-  const int w = padded_head_dim(a.D);
-  if (a.dtype == kBF16)
-    return w == 32 ? launch_main_d<32, true>(a) : w == 64 ? launch_main_d<64, true>(a)
-         : w == 96 ? launch_main_d<96, true>(a) : w == 128 ? launch_main_d<128, true>(a)
-         : launch_main_d<256, true>(a);
-  return w == 32 ? launch_main_d<32, false>(a) : w == 64 ? launch_main_d<64, false>(a)
-       : w == 96 ? launch_main_d<96, false>(a) : w == 128 ? launch_main_d<128, false>(a)
-       : launch_main_d<256, false>(a);
+template <>
+hipError_t launch_bwd_main_w<FA_WIDTH, FA_BF>(const BwdArgs& a) {
+  return launch_main_d<FA_WIDTH, FA_BF>(a);
 }
 
 }  // namespace fa

@@ -250,7 +250,7 @@ int fa_fwd_ex(const void* q, const void* k, const void* v, void* o, float* lse, 
 
 size_t fa_bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D) {
   if (check_shape(B, Hq, Hkv, N, D) != FA_OK) return 0;
-  return fa::bwd_workspace(B, Hq, Hkv, N, D).total;
+  return fa::bwd_workspace_bytes(B, Hq, Hkv, N, D);
 }
 
 static int bwd_pre(const void* dO, const void* o, const float* lse, void* workspace,
@@ -260,9 +260,8 @@ static int bwd_pre(const void* dO, const void* o, const float* lse, void* worksp
   if (rc == FA_OK && layout == fa::kBNHD) rc = check_bnhd(Hq, N, D);
   if (rc != FA_OK) return rc;
   if (!dO || !o || !lse || !workspace) return FA_ERR_NULL;
-  // The vectors and counters this writes lie before the slots, whose offset
-  // depends on neither Hkv nor D.
-  const fa::BwdWorkspace w = fa::bwd_workspace(B, Hq, Hq, N, D);
+  // The vectors and counters this writes lie before the slots.
+  const fa::BwdWorkspace w = fa::bwd_workspace(B, Hq, N);
   if (workspace_bytes < w.slots) return FA_ERR_WORKSPACE;
   char* ws = static_cast<char*>(workspace);
   fa::BwdArgs a{};
@@ -291,6 +290,8 @@ int fa_bwd_preprocess(const void* dO, const void* o, const float* lse, void* wor
 }
 
 // Shared by the main-kernel entry points: fp32 dq or 16-bit dq16.
+// workspace_bytes: kChecked where the caller has compared it.
+static constexpr size_t kChecked = SIZE_MAX;
 static int bwd_main(const void* q, const void* k, const void* v, const void* dO,
                     void* workspace, size_t workspace_bytes, float* dq, void* dq16,
                     void* dk, void* dv, int B, int Hq, int Hkv, int N, int D, int causal,
@@ -301,8 +302,9 @@ static int bwd_main(const void* q, const void* k, const void* v, const void* dO,
   if (rc == FA_OK) rc = check_kv_rows(op, B, Hq, Hkv, N, D);
   if (rc != FA_OK) return rc;
   if (!q || !k || !v || !dO || !workspace || !(dq || dq16) || !dk || !dv) return FA_ERR_NULL;
-  const fa::BwdWorkspace w = fa::bwd_workspace(B, Hq, Hkv, N, D);
-  if (workspace_bytes < w.total) return FA_ERR_WORKSPACE;
+  if (workspace_bytes != kChecked && workspace_bytes < fa::bwd_workspace_bytes(B, Hq, Hkv, N, D))
+    return FA_ERR_WORKSPACE;
+  const fa::BwdWorkspace w = fa::bwd_workspace(B, Hq, N);
   char* ws = static_cast<char*>(workspace);
   fa::BwdArgs a{};
   a.q = q;
@@ -362,7 +364,7 @@ static int bwd_16(const void* q, const void* k, const void* v, const void* dO, c
   if (workspace_bytes < fa_bwd_workspace_bytes(B, Hq, Hkv, N, D)) return FA_ERR_WORKSPACE;
   rc = bwd_pre(dO, o, lse, workspace, workspace_bytes, B, Hq, N, D, op.layout, op.dtype, stream);
   if (rc != FA_OK) return rc;
-  return bwd_main(q, k, v, dO, workspace, workspace_bytes, nullptr, dq, dk, dv, B, Hq, Hkv, N, D,
+  return bwd_main(q, k, v, dO, workspace, kChecked, nullptr, dq, dk, dv, B, Hq, Hkv, N, D,
                   causal, op, stream);
 }
 
@@ -410,8 +412,9 @@ int fa_bwd(const void* q, const void* k, const void* v, const void* dO, const vo
   if (workspace_bytes < fa_bwd_workspace_bytes(B, Hq, Hkv, N, D)) return FA_ERR_WORKSPACE;
   int e = fa_bwd_preprocess(dO, o, lse, workspace, workspace_bytes, B, Hq, N, D, stream);
   if (e != FA_OK) return e;
-  return fa_bwd_main(q, k, v, dO, workspace, workspace_bytes, dq, dk, dv, B, Hq, Hkv, N, D,
-                     causal, stream);
+  if (!dq) return FA_ERR_NULL;
+  return bwd_main(q, k, v, dO, workspace, kChecked, dq, nullptr, dk, dv, B, Hq, Hkv, N, D, causal,
+                  kDefaultOpts, stream);
 }
 
 int fa_pack_mask(const uint8_t* dense, int P, int N, uint32_t* bits, uint32_t* bits_t,
@@ -480,12 +483,17 @@ int fa_bwd_noalloc(const void* q, const void* k, const void* v, const void* dO, 
   a.lse = lse;
   // Both vectors are written in full by the preprocess before the main kernel
   // reads them, so nothing in the scratch needs clearing between calls. No
-  // counters or slots: the main kernel runs without the causal split.
+  // counters: the main kernel runs without the causal split. Slots for key
+  // tiles that several workgroups share, where the rest of the scratch holds them.
   a.dvec = ws;
   a.lse2 = ws + vec / sizeof(float);
   a.counters = nullptr;
   a.n_counters = 0;
-  a.slots = nullptr;
+  const size_t slots = (size_t)fa::bwd_plan(B, Hq, Hkv, N, N, D, causal != 0, D > 32 && D <= 64,
+                                            true).parts *
+                       B * Hkv * ((N + fa::kBwdTile - 1) / fa::kBwdTile) *
+                       fa::bwd_slot_floats(D) * sizeof(float);
+  a.slots = 2 * vec + slots <= kScratchBytes ? ws + 2 * vec / sizeof(float) : nullptr;
   a.dq = dq;
   a.B = B;
   a.Hq = Hq;

@@ -761,22 +761,10 @@ hipError_t launch_fwd_d(const FwdArgs& a) {
 
 }  // namespace
 
-unsigned long long fwd_launch_items(int B, int Hq, int N, int D) {
-  (void)D;
-  const unsigned long long tiles = ((unsigned long long)N + kBR - 1) / kBR;  // non-causal grid
-  const unsigned long long wgs = tiles * (unsigned long long)B * (unsigned long long)Hq;
-  return (wgs + kXcds - 1) / kXcds * kXcds * (padded_head_dim(D) > 128 ? 256 : 512);
-}
-
-hipError_t launch_fwd(const FwdArgs& a) {
-  const int w = padded_head_dim(a.D);
-  if (a.dtype == kBF16)
-    return w == 32 ? launch_fwd_d<32, true>(a) : w == 64 ? launch_fwd_d<64, true>(a)
-         : w == 96 ? launch_fwd_d<96, true>(a) : w == 128 ? launch_fwd_d<128, true>(a)
-                                                         : launch_fwd_d<256, true>(a);
-  return w == 32 ? launch_fwd_d<32, false>(a) : w == 64 ? launch_fwd_d<64, false>(a)
-       : w == 96 ? launch_fwd_d<96, false>(a) : w == 128 ? launch_fwd_d<128, false>(a)
-                                                         : launch_fwd_d<256, false>(a);
+// One object file per width and format (-DFA_WIDTH, -DFA_BF), compiled in parallel.
+template <>
+hipError_t launch_fwd_w<FA_WIDTH, FA_BF>(const FwdArgs& a) {
+  return launch_fwd_d<FA_WIDTH, FA_BF>(a);
 }
 
 }  // namespace fa

@@ -86,7 +86,8 @@ inline int key_rows(int N, int Nkv) { return Nkv > 0 ? Nkv : N; }
 //   one counter per pair of key tiles (u, n_tiles-1-u) per (b, head), which
 //   the preprocess kernel zeroes (sized by Hq, which bounds Hkv, so that the
 //   preprocess needs no Hkv);
-//   two fp32 partial dK/dV slots per such pair and (b, kv head).
+//   fp32 partial dK/dV slots: two per such pair and (b, kv head), or, where
+//   several workgroups share a key tile (BwdPlan::parts), one for each of them.
 // Head dims: any multiple of 8 from 8 to 256 (the `D` of the argument
 // structs, the row length in memory). The kernels are compiled for the
 // widths 32, 64, 96, 128 and 256 and run a head dim on the smallest that
@@ -97,15 +98,28 @@ inline int padded_head_dim(int D) {
 inline bool valid_head_dim(int D) { return D >= 8 && D <= 256 && D % 8 == 0; }
 
 constexpr int kBwdTile = 128;  // key rows of one backward workgroup
+
+// How the backward's main kernel divides its work (bwd_plan, fa_launch.hip).
+struct BwdPlan {
+  bool apart;  // the two phases as work items of their own
+  int parts;   // (apart) workgroups that share one key tile's phase 1
+  bool w4;     // width 64: the two-workgroups-per-CU shape
+};
+// has_w4: the launch has such an instantiation; slots: it has the slots of
+// bwd_workspace for NK == N.
+BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, bool has_w4,
+                 bool slots);
+// The most parts bwd_plan takes for a shape, whatever the call's options.
+int bwd_max_parts(int B, int Hq, int Hkv, int N, int D);
 struct BwdWorkspace {
-  size_t dvec, lse2, counters, slots, total;
+  size_t dvec, lse2, counters, slots;
   int n_counters;
 };
 inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 inline size_t bwd_slot_floats(int D) {  // dK^T, dV^T at the padded width
   return (size_t)kBwdTile * padded_head_dim(D) * 2;
 }
-inline BwdWorkspace bwd_workspace(int B, int Hq, int Hkv, int N, int D) {
+inline BwdWorkspace bwd_workspace(int B, int Hq, int N) {
   BwdWorkspace w;
   const size_t vec = align256((size_t)B * Hq * N * sizeof(float));
   const int pairs_per_head = ((N + kBwdTile - 1) / kBwdTile) / 2;
@@ -114,8 +128,16 @@ inline BwdWorkspace bwd_workspace(int B, int Hq, int Hkv, int N, int D) {
   w.counters = 2 * vec;
   w.n_counters = B * Hq * pairs_per_head;
   w.slots = w.counters + align256((size_t)w.n_counters * sizeof(unsigned));
-  w.total = w.slots + (size_t)B * Hkv * pairs_per_head * 2 * bwd_slot_floats(D) * sizeof(float);
   return w;
+}
+inline size_t bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D) {
+  const int pairs_per_head = ((N + kBwdTile - 1) / kBwdTile) / 2;
+  // Slots: two per pair (the causal split), or one per part of each key tile.
+  const int parts = bwd_max_parts(B, Hq, Hkv, N, D);
+  size_t per_head = (size_t)pairs_per_head * 2;
+  if (parts > 1) per_head = (size_t)parts * ((N + kBwdTile - 1) / kBwdTile);
+  return bwd_workspace(B, Hq, N).slots +
+         (size_t)B * Hkv * per_head * bwd_slot_floats(D) * sizeof(float);
 }
 
 struct BwdArgs {
@@ -137,9 +159,8 @@ struct BwdArgs {
   int layout = kBHND;  // of q, k, v, dO, o, dq, dk, dv (lse, workspace dense)
   unsigned* counters = nullptr;  // workspace: per key-tile pair (zeroed by the preprocess)
   int n_counters = 0;
-  // Workspace: partial dK/dV of split key tiles. Null turns the causal split
-  // off (every key tile's phase 1 stays in its own workgroup), so neither the
-  // slots nor the counters are touched.
+  // Workspace: partial dK/dV of shared key tiles. Null: every key tile's phase
+  // 1 stays in its own workgroup. Null counters turn the causal split off.
   float* slots = nullptr;
   int dtype = kFP16;             // of q, k, v, dO, o, dk, dv and dq16
   const int* kv_len = nullptr;   // as FwdArgs::kv_len
@@ -172,6 +193,14 @@ struct BwdArgs {
   const int* block_cols = nullptr;
 };
 
+// The launches of tile width W and format (BF: bf16), an object file each, and
+// the ones that pick them (fa_launch.hip).
+template <int W, bool BF>
+hipError_t launch_fwd_w(const FwdArgs& a);
+template <int W, bool BF>
+hipError_t launch_bwd_pre_w(const BwdArgs& a);
+template <int W, bool BF>
+hipError_t launch_bwd_main_w(const BwdArgs& a);
 hipError_t launch_fwd(const FwdArgs& a);
 hipError_t launch_bwd_preprocess(const BwdArgs& a);
 hipError_t launch_bwd_main(const BwdArgs& a);

@@ -379,8 +379,9 @@ int fa_pack_blocks(const uint8_t* layout, int layout_b, int layout_h, int B, int
  * the process ends), so the shape must satisfy 2 * align256(B*Hq*N*4) <=
  * FA_BWD_NOALLOC_SCRATCH_BYTES (B*Hq*N <= 2^21 rows), else FA_ERR_SCRATCH and
  * nothing is launched. The causal load balancing that needs workspace slots is
- * off, so dk and dv may differ from fa_bwd's in the last bits (dq is the same);
- * results are deterministic. `stream` must belong to the current device.
+ * off, and key tiles are shared by several workgroups only where their partial
+ * sums fit the array too, so dk and dv may differ from fa_bwd's in the last bits
+ * (dq is the same); results are deterministic. `stream` must belong to the current device.
  * Every call on a GPU shares that GPU's scratch: calls that overlap in time
  * on one GPU (other streams, other host threads) race and give wrong results;
  * calls ordered on one stream are fine.

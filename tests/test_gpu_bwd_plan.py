@@ -1,0 +1,82 @@
+"""The backward's work division (bwd_plan, csrc/fa_launch.hip): phases apart,
+key tiles shared by several workgroups, two workgroups per CU and one item per
+tile, each at shapes whose plan takes it, with ragged edges, against the
+float64 oracle at the suite's bars. No counterpart in the reference, which has
+one backward grid (flash_bwd.cuh:475-483)."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import FWD_MAX_ABS, GRAD_REL_L2, REF_REL, make_inputs, np64
+from oracle import attention as ora
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+CASES = [
+    # B, Hq, Hkv, N, D, causal
+    (1, 4, 4, 256, 64, True),     # apart, one part
+    (1, 16, 1, 385, 64, True),    # parts: one kv head, a ragged last tile
+    (1, 16, 1, 511, 128, False),  # parts, dense ragged (keys past N masked once)
+    (1, 6, 2, 129, 128, True),    # a tile of one row; more parts than steps in it
+    (2, 4, 2, 300, 256, True),    # parts at width 256
+    (1, 8, 2, 300, 96, True),     # parts at width 96
+    (1, 8, 2, 200, 40, False),    # a head dim below its width
+    (3, 12, 12, 700, 64, False),  # two workgroups per CU, apart
+    (9, 8, 8, 537, 128, True),    # over one round of one item per tile, apart
+    (1, 1, 1, 2, 128, True),      # two rows (with one, dQ and dK are zero up to rounding)
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal", CASES)
+def test_plans_match_oracle(B, Hq, Hkv, N, D, causal):
+    import fa_p100
+    q, k, v, do = make_inputs(B, Hq, Hkv, N, D, seed=N + D)
+    qg, kg, vg = (t.to(DEV).requires_grad_(True) for t in (q, k, v))
+    o = fa_p100.flash_attn(qg, kg, vg, causal)
+    grads = torch.autograd.grad(o, (qg, kg, vg), do.to(DEV), retain_graph=True)
+    again = torch.autograd.grad(o, (qg, kg, vg), do.to(DEV))
+    G = Hq // Hkv
+    b = B - 1  # one batch entry and its last kv head's group
+    sq, sk = (slice(b, B), slice(Hq - G, Hq)), (slice(b, B), slice(Hkv - 1, Hkv))
+    args = [np64(t) for t in (q[sq], k[sk], v[sk])]
+    ref = ora.attention_bwd(*args, np64(do[sq]), causal)
+    assert ora.max_abs(np64(o[sq]), ora.attention_fwd(*args, causal)[0]) <= FWD_MAX_ABS
+    for name, g, r, s in zip(("dQ", "dK", "dV"), grads, ref, (sq, sk, sk)):
+        g = np64(g[s])
+        assert np.isfinite(g).all(), name
+        assert ora.rel_max_rms(g, r) < REF_REL if np.any(r) else not np.any(g), name
+        if np.any(r):
+            assert ora.rel_l2(g, r) <= GRAD_REL_L2, name
+    for g, h in zip(grads, again):  # the parts are added in one order
+        assert torch.equal(g, h)
+
+
+def test_key_tiles_past_every_key_length_have_zero_gradients():
+    """Key tiles wholly past an entry's key length run no step; their dK, dV
+    are written as zeros, in every plan."""
+    import fa_p100
+    B, H, N, D = 2, 2, 640, 64
+    q, k, v, do = (t.to(DEV) for t in make_inputs(B, H, H, N, D, seed=3))
+    kv_len = torch.tensor([130, 640], dtype=torch.int32, device=DEV)
+    for causal in (False, True):
+        leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        fa_p100.flash_attn(*leaves, causal, kv_len=kv_len).backward(do)
+        for g in (leaves[1].grad, leaves[2].grad):
+            assert torch.isfinite(g).all() and not g[0, :, 130:].any()
+            assert g[0, :, :130].any() and g[1, :, 512:].any()
+
+
+def test_shared_tiles_with_nan_workspace():
+    """Slots and outputs hold NaN before the call: every value read was written."""
+    import fa_p100
+    q, k, v, do = (t.to(DEV) for t in make_inputs(1, 16, 1, 500, 64, seed=4))
+    o, lse = fa_p100._ext.forward_dt(q, k, v, True)
+    ref = fa_p100._ext.backward_dt(q, k, v, do, o, lse, True)
+    junk = torch.full((64 << 20,), float("nan"), device=DEV)
+    torch.cuda.synchronize()
+    del junk  # its block serves the next call's workspace
+    got = fa_p100._ext.backward_dt(q, k, v, do, o, lse, True)
+    for a, b in zip(got, ref):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
