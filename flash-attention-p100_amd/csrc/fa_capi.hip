@@ -189,15 +189,15 @@ static uint32_t dropout_threshold(float p) {
   return (uint32_t)(t < 0.0 ? 0.0 : t > 65535.0 ? 65535.0 : t);
 }
 
-static int fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B, int Hq,
-               int Hkv, int N, int D, int causal, const fa_options& op, void* stream) {
+// Checks a forward call and fills its arguments.
+static int fwd_args(const void* q, const void* k, const void* v, void* o, float* lse, int B, int Hq,
+                    int Hkv, int N, int D, int causal, const fa_options& op, void* stream,
+                    fa::FwdArgs& a) {
   int rc = check_opts(op, causal, Hq, N, D, false);
   if (rc == FA_OK) rc = check_shape(B, Hq, Hkv, N, D);
   if (rc == FA_OK && op.layout == fa::kBNHD) rc = check_bnhd(Hq, N, D);
   if (rc == FA_OK) rc = check_kv_rows(op, B, Hq, Hkv, N, D);
   if (rc != FA_OK) return rc;
-  if (!q || !k || !v || !o || !lse) return FA_ERR_NULL;
-  fa::FwdArgs a{};
   a.q = q;
   a.k = k;
   a.v = v;
@@ -227,7 +227,19 @@ static int fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   a.bias_sh = op.bias_stride_h;
   a.Nkv = op.kv_rows;
   a.block_rows = op.block_rows;
-  return to_code(fa::launch_fwd(a));
+  return FA_OK;
+}
+
+static int fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B, int Hq,
+               int Hkv, int N, int D, int causal, const fa_options& op, void* stream,
+               void* workspace = nullptr, size_t workspace_bytes = 0) {
+  fa::FwdArgs a{};
+  const int rc = fwd_args(q, k, v, o, lse, B, Hq, Hkv, N, D, causal, op, stream, a);
+  if (rc != FA_OK) return rc;
+  if (!q || !k || !v || !o || !lse) return FA_ERR_NULL;
+  if (workspace && workspace_bytes < fa::dec_workspace_bytes(fa::dec_plan(a), D))
+    return FA_ERR_WORKSPACE;
+  return to_code(fa::launch_fwd(a, workspace));
 }
 
 int fa_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B, int Hq,
@@ -246,6 +258,22 @@ int fa_fwd_bnhd(const void* q, const void* k, const void* v, void* o, float* lse
 int fa_fwd_ex(const void* q, const void* k, const void* v, void* o, float* lse, int B, int Hq,
               int Hkv, int N, int D, int causal, const fa_options* opts, void* stream) {
   return fwd(q, k, v, o, lse, B, Hq, Hkv, N, D, causal, opts ? *opts : kDefaultOpts, stream);
+}
+
+size_t fa_fwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int causal,
+                              const fa_options* opts) {
+  fa::FwdArgs a{};
+  if (fwd_args(nullptr, nullptr, nullptr, nullptr, nullptr, B, Hq, Hkv, N, D, causal,
+               opts ? *opts : kDefaultOpts, nullptr, a) != FA_OK)
+    return 0;
+  return fa::dec_workspace_bytes(fa::dec_plan(a), D);
+}
+
+int fa_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,
+              size_t workspace_bytes, int B, int Hq, int Hkv, int N, int D, int causal,
+              const fa_options* opts, void* stream) {
+  return fwd(q, k, v, o, lse, B, Hq, Hkv, N, D, causal, opts ? *opts : kDefaultOpts, stream,
+             workspace, workspace_bytes);
 }
 
 size_t fa_bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D) {

@@ -146,7 +146,56 @@ int bwd_max_parts(int B, int Hq, int Hkv, int N, int D) {
   return most;
 }
 
-hipError_t launch_fwd(const FwdArgs& a) {
+// Estimated microseconds, fitted to 20 shapes (1 to 512 query rows, 1000 to
+// 32768 keys): a workgroup of fa_dec.hip takes 1.2 us for a round of its waves
+// (256 keys; 128 at width 256) while it waits for memory and 1.5 where every CU
+// has one, 2 us to start and end; the keys and values come at 5.4 TB/s; parts
+// cost a second launch (2 us on the GPU, 3 on the host, which small calls wait
+// for) and 0.019 us for each partial O (width 128) to write and
+// combine. A step (128 keys) of fa_fwd.hip takes 1 us.
+// Same box, fa_fwd.hip -> here: 220 -> 99 us at B=16 H=32/8 N=1 against 8192
+// keys, D=128 (2 parts); 238 -> 29 at B=1 H=32/8 N=1, 32768 keys, D=128 (16
+// parts); 225 -> 18 at B=1 H=16/2 N=4, 8000 keys, D=256 (16 parts); 55 -> 23 at
+// B=32 H=32/8 N=1, 1000 keys, D=128 (1 part); 68 -> 23 at B=1 H=32/8 N=128, 4096
+// keys, D=128 (2 parts); 71 -> 76 at B=4 H=32/4 N=321, 1506 keys, D=128, which
+// stays there. Only with more keys than query rows: the square shapes' results
+// do not change.
+DecPlan dec_plan(const FwdArgs& a) {
+  constexpr int kTried[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+  const DecPlan none{0, 0, 1};
+  const int NK = key_rows(a.N, a.Nkv), W = padded_head_dim(a.D);
+  if (NK <= a.N || a.mask || a.drop || a.bias || a.block_rows || a.seg_start) return none;
+  const double tiles = ceil((double)(a.Hq / a.Hkv) * a.N / 32), items = tiles * a.B * a.Hkv;
+  if (items * 512 > 4294967295.0 || items * (W / 32) * 256 > 4294967295.0) return none;
+  const int wave_keys = W > 128 ? 128 : 256;
+  const double seen = a.window > 0 ? fmin(NK, (double)a.window + a.N) : NK;
+  const double read = 4.0 * a.B * a.Hkv * seen * a.D / 5.4e6;
+  double least = HUGE_VAL;
+  int best = 1;
+  for (const int parts : kTried) {
+    if (parts > 1 && (seen < parts * 128.0 || items * parts > 4096)) break;
+    const double rounds = ceil(items * parts / kCUs);
+    const double each = ceil(seen / parts / wave_keys) * (items * parts >= kCUs ? 1.5 : 1.2) + 2.0;
+    const double t = fmax(rounds * each, read) + (parts > 1 ? 5.0 + 0.019 * items * parts * W / 128 : 0.0);
+    if (t < least) {
+      least = t;
+      best = parts;
+    }
+  }
+  const double q_tiles = (a.N + 63) / 64, per_wg = a.causal && q_tiles > 1 ? 2 : 1;
+  const double wgs = ceil(q_tiles / per_wg) * a.B * a.Hq;
+  const double there = ceil(wgs / kCUs) * per_wg * (seen / (W > 128 ? 64 : 128) + 2.0);
+  return least < there ? DecPlan{(int)tiles, (int)items, best} : none;
+}
+
+hipError_t launch_fwd(const FwdArgs& a, void* workspace) {
+  DecPlan plan = dec_plan(a);
+  if (plan.items > 0) {
+    if (!workspace) plan.parts = 1;
+    return by_width(a, a.dtype == kBF16, [&](auto w, auto bf, const FwdArgs& a) {
+      return launch_dec_w<decltype(w)::value, decltype(bf)::value>(a, plan, workspace);
+    });
+  }
   return by_width(a, a.dtype == kBF16, [](auto w, auto bf, const FwdArgs& a) {
     return launch_fwd_w<decltype(w)::value, decltype(bf)::value>(a);
   });

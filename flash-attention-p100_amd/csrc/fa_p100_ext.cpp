@@ -208,6 +208,19 @@ std::vector<at::Tensor> fa_forward(at::Tensor q, at::Tensor k, at::Tensor v, boo
   return {o, lse};
 }
 
+// fa_fwd_ws with a workspace from torch's allocator where the call needs one.
+static void forward_ws(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                       const at::Tensor& o, const at::Tensor& lse, int B, int H, int Hkv, int N,
+                       int D, bool causal, const fa_options& op) {
+  const size_t bytes = fa_fwd_workspace_bytes(B, H, Hkv, N, D, causal ? 1 : 0, &op);
+  at::Tensor ws;
+  if (bytes) ws = at::empty({(int64_t)bytes}, q.options().dtype(at::kByte));
+  check_rc(fa_fwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(),
+                     bytes ? ws.data_ptr() : nullptr, bytes, B, H, Hkv, N, D, causal ? 1 : 0, &op,
+                     current_stream(q)),
+           "fa_fwd_ws");
+}
+
 // half_dq: dq comes back as fp16 (the fp32 result rounded to nearest even,
 // bit-identical to casting the fp32 dq) for the autograd backward, which
 // returns dq in q's dtype (fa_p100.py:45); otherwise fp32 as the reference.
@@ -318,10 +331,7 @@ std::vector<at::Tensor> fa_forward_bnhd(at::Tensor q, at::Tensor k, at::Tensor v
                 B, H, Hkv, N);
   // key rows that differ from the query rows: bottom-right-aligned causal
   op.kv_rows = k.size(1) != N ? (int)k.size(1) : 0;
-  check_rc(fa_fwd_ex(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                     lse.data_ptr<float>(), B, H, Hkv, N, D, causal ? 1 : 0, &op,
-                     current_stream(q)),
-           "fa_fwd_ex");
+  forward_ws(q, k, v, o, lse, B, H, Hkv, N, D, causal, op);
   return {o, lse};
 }
 
@@ -414,10 +424,7 @@ std::vector<at::Tensor> fa_forward_dt(at::Tensor q, at::Tensor k, at::Tensor v, 
                 B, H, Hkv, N);
   // key rows that differ from the query rows: bottom-right-aligned causal
   op.kv_rows = k.size(2) != N ? (int)k.size(2) : 0;
-  check_rc(fa_fwd_ex(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                     lse.data_ptr<float>(), B, H, Hkv, N, D, causal ? 1 : 0, &op,
-                     current_stream(q)),
-           "fa_fwd_ex");
+  forward_ws(q, k, v, o, lse, B, H, Hkv, N, D, causal, op);
   return {o, lse};
 }
 

@@ -308,6 +308,22 @@ typedef struct fa_options {
 int fa_fwd_ex(const void* q, const void* k, const void* v, void* o, float* lse,
               int B, int Hq, int Hkv, int N, int D, int causal, const fa_options* opts,
               void* stream);
+
+/*
+ * fa_fwd_ex with a workspace: a call over few query rows (KV-cache decoding,
+ * a short chunk behind a long cache) then shares each row's keys among several
+ * workgroups, whose partial results meet in the workspace. `workspace` holds
+ * at least fa_fwd_workspace_bytes() bytes for the same arguments (0 for the
+ * calls that need none: any pointer, or NULL, will do) and may hold anything;
+ * calls that overlap in time need workspaces of their own. With NULL this is
+ * fa_fwd_ex. Results differ from fa_fwd_ex's in the last bits. No counterpart
+ * in the reference.
+ */
+size_t fa_fwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int causal,
+                              const fa_options* opts);
+int fa_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,
+              size_t workspace_bytes, int B, int Hq, int Hkv, int N, int D, int causal,
+              const fa_options* opts, void* stream);
 int fa_bwd_ex(const void* q, const void* k, const void* v, const void* dO, const void* o,
               const float* lse, void* dq, void* dk, void* dv, void* workspace,
               size_t workspace_bytes, int B, int Hq, int Hkv, int N, int D, int causal,
