@@ -26,7 +26,7 @@ LIB_NAME = "libfa_mi355x.so"
 EXT_NAME = "fa_p100_ext"
 KERNEL_SOURCES = ["fa_launch.hip", "fa_mask.hip", "fa_capi.hip"]
 # Compiled once per tile width and format (-DFA_WIDTH, -DFA_BF), the slowest first.
-WIDTH_SOURCES = ["fa_bwd.hip", "fa_fwd.hip", "fa_dec.hip"]
+WIDTH_SOURCES = ["fa_bwd.hip", "fa_fwd.hip", "fa_rows.hip", "fa_dec.hip"]
 WIDTHS = [128, 96, 64, 256, 32]
 
 HIPCC_FLAGS = [

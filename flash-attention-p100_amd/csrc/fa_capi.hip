@@ -237,7 +237,7 @@ static int fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   const int rc = fwd_args(q, k, v, o, lse, B, Hq, Hkv, N, D, causal, op, stream, a);
   if (rc != FA_OK) return rc;
   if (!q || !k || !v || !o || !lse) return FA_ERR_NULL;
-  if (workspace && workspace_bytes < fa::dec_workspace_bytes(fa::dec_plan(a), D))
+  if (workspace && workspace_bytes < fa::fwd_workspace_bytes(fa::fwd_plan(a), D))
     return FA_ERR_WORKSPACE;
   return to_code(fa::launch_fwd(a, workspace));
 }
@@ -266,7 +266,7 @@ size_t fa_fwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int causal,
   if (fwd_args(nullptr, nullptr, nullptr, nullptr, nullptr, B, Hq, Hkv, N, D, causal,
                opts ? *opts : kDefaultOpts, nullptr, a) != FA_OK)
     return 0;
-  return fa::dec_workspace_bytes(fa::dec_plan(a), D);
+  return fa::fwd_workspace_bytes(fa::fwd_plan(a), D);
 }
 
 int fa_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,

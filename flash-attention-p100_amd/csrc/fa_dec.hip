@@ -291,9 +291,7 @@ __global__ __launch_bounds__(256) void dec_merge_kernel(const DecArgs a) {
 
 }  // namespace
 
-template <>
-hipError_t launch_dec_w<FA_WIDTH, FA_BF>(const FwdArgs& a, const DecPlan& plan, void* workspace) {
-  constexpr int D = FA_WIDTH;
+static DecArgs dec_args(const FwdArgs& a, const FwdPlan& plan, void* workspace) {
   DecArgs d{};
   d.q = (const half_t*)a.q;
   d.k = (const half_t*)a.k;
@@ -317,13 +315,29 @@ hipError_t launch_dec_w<FA_WIDTH, FA_BF>(const FwdArgs& a, const DecPlan& plan, 
   d.stk = make_strides(a.layout, a.Hkv, d.NK, a.D);
   if (plan.parts > 1) {
     d.part_ml = (float2*)workspace;
-    d.part_o = (float*)((char*)workspace + dec_ml_bytes(plan));
+    d.part_o = (float*)((char*)workspace + part_ml_bytes(plan));
   }
+  return d;
+}
+
+template <>
+hipError_t launch_dec_w<FA_WIDTH, FA_BF>(const FwdArgs& a, const FwdPlan& plan, void* workspace) {
+  constexpr int D = FA_WIDTH;
+  const DecArgs d = dec_args(a, plan, workspace);
   hipLaunchKernelGGL((dec_kernel<D, FA_BF>), dim3((unsigned)xcd_grid(plan.items * plan.parts)),
                      dim3(Dec<D>::kThreads), 0, (hipStream_t)a.stream, d);
-  if (plan.parts > 1)
-    hipLaunchKernelGGL((dec_merge_kernel<D, FA_BF>), dim3((unsigned)plan.items * (D / 32)),
-                       dim3(256), 0, (hipStream_t)a.stream, d);
+  return hipGetLastError();
+}
+
+// Combines the parts of fa_rows.hip's row blocks (each a head's own: group 1)
+// or of this file's row tiles.
+template <>
+hipError_t launch_merge_w<FA_WIDTH, FA_BF>(const FwdArgs& a, const FwdPlan& plan, void* workspace) {
+  constexpr int D = FA_WIDTH;
+  DecArgs d = dec_args(a, plan, workspace);
+  if (plan.kind == FwdPlan::kRows) d.group = 1;
+  hipLaunchKernelGGL((dec_merge_kernel<D, FA_BF>), dim3((unsigned)plan.items * (D / 32)), dim3(256),
+                     0, (hipStream_t)a.stream, d);
   return hipGetLastError();
 }
 

@@ -193,21 +193,23 @@ struct BwdArgs {
   const int* block_cols = nullptr;
 };
 
-// Forward over few query rows (fa_dec.hip): row tiles per kv head, row tiles in
-// all, and the workgroups that share a row tile's keys. items == 0: the call
-// runs on fa_fwd.hip instead.
-struct DecPlan {
-  int tiles, items, parts;
+// Which kernel a forward call runs on (fwd_plan, fa_launch.hip).
+struct FwdPlan {
+  enum Kind { kTiles, kRows, kDec } kind;  // fa_fwd.hip, fa_rows.hip, fa_dec.hip
+  int waves;  // (kRows) of a workgroup
+  bool pair;  // (kRows) a workgroup takes a long and a short causal tile
+  int parts;  // (kRows, kDec) workgroups that share a row block's keys
+  // 32-row blocks whose partial results the parts write: per head (kRows) or
+  // kv head (kDec), and in all.
+  int tiles, items;
 };
-// Whether and how a call runs on fa_dec.hip; parts are for a workspace of
-// dec_workspace_bytes.
-DecPlan dec_plan(const FwdArgs& a);
-inline size_t dec_ml_bytes(const DecPlan& p) {  // (max, sum) per row of each part
+FwdPlan fwd_plan(const FwdArgs& a);
+inline size_t part_ml_bytes(const FwdPlan& p) {  // (max, sum) per row of each part
   return align256((size_t)p.items * p.parts * 32 * 8);
 }
-inline size_t dec_workspace_bytes(const DecPlan& p, int D) {
+inline size_t fwd_workspace_bytes(const FwdPlan& p, int D) {
   if (p.parts <= 1) return 0;
-  return dec_ml_bytes(p) + (size_t)p.items * p.parts * 32 * padded_head_dim(D) * sizeof(float);
+  return part_ml_bytes(p) + (size_t)p.items * p.parts * 32 * padded_head_dim(D) * sizeof(float);
 }
 
 // The launches of tile width W and format (BF: bf16), an object file each, and
@@ -215,12 +217,16 @@ inline size_t dec_workspace_bytes(const DecPlan& p, int D) {
 template <int W, bool BF>
 hipError_t launch_fwd_w(const FwdArgs& a);
 template <int W, bool BF>
-hipError_t launch_dec_w(const FwdArgs& a, const DecPlan& plan, void* workspace);
+hipError_t launch_rows_w(const FwdArgs& a, const FwdPlan& plan, void* workspace);
+template <int W, bool BF>
+hipError_t launch_dec_w(const FwdArgs& a, const FwdPlan& plan, void* workspace);
+template <int W, bool BF>
+hipError_t launch_merge_w(const FwdArgs& a, const FwdPlan& plan, void* workspace);
 template <int W, bool BF>
 hipError_t launch_bwd_pre_w(const BwdArgs& a);
 template <int W, bool BF>
 hipError_t launch_bwd_main_w(const BwdArgs& a);
-// workspace: dec_workspace_bytes(dec_plan(a)) bytes, or null (no parts).
+// workspace: fwd_workspace_bytes(fwd_plan(a)) bytes, or null (no parts).
 hipError_t launch_fwd(const FwdArgs& a, void* workspace);
 hipError_t launch_bwd_preprocess(const BwdArgs& a);
 hipError_t launch_bwd_main(const BwdArgs& a);

@@ -146,58 +146,161 @@ int bwd_max_parts(int B, int Hq, int Hkv, int N, int D) {
   return most;
 }
 
-// Estimated microseconds, fitted to 20 shapes (1 to 512 query rows, 1000 to
-// 32768 keys): a workgroup of fa_dec.hip takes 1.2 us for a round of its waves
-// (256 keys; 128 at width 256) while it waits for memory and 1.5 where every CU
-// has one, 2 us to start and end; the keys and values come at 5.4 TB/s; parts
-// cost a second launch (2 us on the GPU, 3 on the host, which small calls wait
-// for) and 0.019 us for each partial O (width 128) to write and
-// combine. A step (128 keys) of fa_fwd.hip takes 1 us.
-// Same box, fa_fwd.hip -> here: 220 -> 99 us at B=16 H=32/8 N=1 against 8192
-// keys, D=128 (2 parts); 238 -> 29 at B=1 H=32/8 N=1, 32768 keys, D=128 (16
-// parts); 225 -> 18 at B=1 H=16/2 N=4, 8000 keys, D=256 (16 parts); 55 -> 23 at
-// B=32 H=32/8 N=1, 1000 keys, D=128 (1 part); 68 -> 23 at B=1 H=32/8 N=128, 4096
-// keys, D=128 (2 parts); 71 -> 76 at B=4 H=32/4 N=321, 1506 keys, D=128, which
-// stays there. Only with more keys than query rows: the square shapes' results
-// do not change.
-DecPlan dec_plan(const FwdArgs& a) {
-  constexpr int kTried[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
-  const DecPlan none{0, 0, 1};
+// Estimated microseconds of a forward on each kernel, fitted per width to 6110
+// random square shapes (100 <= N <= 8192, B <= 16, 1 to 64 heads) and 1359 with
+// up to 16384 more keys than query rows, every candidate timed for each: the
+// plan taken is 1.5% slower than the best candidate on average over the square
+// shapes (5% over the others), fa_fwd.hip alone 39% (95%). Same box, fa_fwd.hip
+// -> the plan's: 349 -> 293 us at B=2 H=32/8 N=3001 D=128 dense (fa_rows.hip, 8
+// waves), 315 -> 280 at B=1 H=16 N=8192 D=128 causal (8 waves), 239 -> 166 at
+// B=9 H=12 N=2145 D=128 causal (4 waves), 21 -> 8.8 at B=14 H=12 N=189 D=64
+// causal; fa_fwd.hip stays where few rows leave CUs idle (B=1 H=8 N=4096 D=128
+// causal: 47 us, 71 with 4 waves). More keys than rows: 220 -> 99 at B=16 H=32/8
+// N=1, 8192 keys, D=128 (fa_dec.hip, 2 parts); 238 -> 29 at B=1 H=32/8 N=1, 32768
+// keys (16 parts); 225 -> 18 at B=1 H=16/2 N=4, 8000 keys, D=256 (16 parts);
+// 141 -> 81 at B=1 H=32/8 N=512, 8192 keys (fa_rows.hip, 8 waves, 4 parts).
+namespace {
+
+// One kernel's times at a width.
+struct FwdTimes {
+  double solo, full;  // a step of a workgroup, alone on its CU and with it full
+  double ends;        // a tile's start and end
+  double uneven;      // (causal fa_rows.hip) the end of the grid, in longest tiles
+  int per_cu;         // workgroups that share a CU
+};
+enum { kW32, kW64, kW96, kW128, kW256 };
+constexpr FwdTimes kTilesTimes[] = {{0.60, 0.70, 4.2, 0, 1}, {0.60, 0.70, 4.2, 0, 1},
+                                    {0.80, 0.95, 4.2, 0, 1}, {0.98, 1.12, 7.0, 0, 1},
+                                    {1.38, 1.38, 20.2, 0, 1}};
+constexpr FwdTimes kRows4Times[] = {{0.69, 2.38, 4.6, 0.25, 4}, {0.69, 2.38, 4.6, 0.25, 4},
+                                    {0.86, 2.28, 4.9, 0.31, 3}, {1.02, 1.93, 5.6, 0.41, 2},
+                                    {2.06, 2.54, 8.7, 0.39, 1}};
+constexpr FwdTimes kRows8Times[] = {{1.03, 2.49, 4.8, 0.25, 2}, {1.03, 2.49, 4.8, 0.25, 2},
+                                    {1.21, 1.63, 4.9, 0.32, 1}, {1.46, 2.11, 6.0, 0.27, 1},
+                                    {2.72, 4.12, 9.5, 0.20, 1}};
+constexpr FwdTimes kPairTimes[] = {{0.80, 2.67, 3.4, 0, 4}, {0.80, 2.67, 3.4, 0, 4},
+                                   {1.21, 2.66, 3.8, 0, 3}, {1.49, 2.24, 4.2, 0, 2},
+                                   {2.96, 3.08, 6.2, 0, 1}};
+// (a round of fa_dec.hip: 256 keys, 128 at width 256)
+constexpr double kDecTimes[] = {0.9, 0.9, 1.3, 1.6, 1.5};
+// Two workgroups per CU of fa_fwd.hip (FwdShape W4): a step on a full chip.
+constexpr double kTilesW4[] = {0, 1.27, 0, 2.2, 0};
+
+double step_time(const FwdTimes& t, double per_cu) {
+  if (t.per_cu == 1) return t.full;
+  const double r = fmin(fmax(per_cu, 1.0), t.per_cu);
+  return t.solo + (t.full - t.solo) * (r - 1) / (t.per_cu - 1);
+}
+// n equal workgroups of `steps` steps and `tiles` tiles.
+double equal_time(const FwdTimes& t, double n, double steps, double tiles) {
+  const double slots = (double)kCUs * t.per_cu, full = floor(n / slots), rest = n - full * slots;
+  double us = full * (steps * t.full + tiles * t.ends);
+  if (rest > 0) us += steps * step_time(t, ceil(rest / kCUs)) + tiles * t.ends;
+  return us;
+}
+// n causal tiles of `total` steps in all, the longest first.
+double uneven_time(const FwdTimes& t, double n, double total, double longest) {
+  const double slots = (double)kCUs * t.per_cu;
+  return fmax(total * t.full / slots + n / slots * t.ends + t.uneven * longest * t.full,
+              longest * step_time(t, ceil(n / kCUs)) + t.ends);
+}
+double ceil_div(double a, double b) { return ceil(a / b); }
+
+}  // namespace
+
+FwdPlan fwd_plan(const FwdArgs& a) {
+  FwdPlan best{FwdPlan::kTiles, 0, false, 1, 0, 0};
+  if (a.mask || a.drop || a.bias || a.block_rows) return best;
   const int NK = key_rows(a.N, a.Nkv), W = padded_head_dim(a.D);
-  if (NK <= a.N || a.mask || a.drop || a.bias || a.block_rows || a.seg_start) return none;
-  const double tiles = ceil((double)(a.Hq / a.Hkv) * a.N / 32), items = tiles * a.B * a.Hkv;
-  if (items * 512 > 4294967295.0 || items * (W / 32) * 256 > 4294967295.0) return none;
-  const int wave_keys = W > 128 ? 128 : 256;
-  const double seen = a.window > 0 ? fmin(NK, (double)a.window + a.N) : NK;
-  const double read = 4.0 * a.B * a.Hkv * seen * a.D / 5.4e6;
-  double least = HUGE_VAL;
-  int best = 1;
-  for (const int parts : kTried) {
-    if (parts > 1 && (seen < parts * 128.0 || items * parts > 4096)) break;
-    const double rounds = ceil(items * parts / kCUs);
-    const double each = ceil(seen / parts / wave_keys) * (items * parts >= kCUs ? 1.5 : 1.2) + 2.0;
-    const double t = fmax(rounds * each, read) + (parts > 1 ? 5.0 + 0.019 * items * parts * W / 128 : 0.0);
-    if (t < least) {
-      least = t;
-      best = parts;
+  const int wi = W <= 32 ? kW32 : W <= 64 ? kW64 : W <= 96 ? kW96 : W <= 128 ? kW128 : kW256;
+  const double BH = (double)a.B * a.Hq, kofs = NK - a.N;
+  // Keys seen by the rows of a tile that ends before row i1, a window's start rounded down.
+  auto keys = [&](double rows, double i1) {
+    const double hi = a.causal ? fmax(1, fmin(NK, i1 + kofs)) : NK;
+    return a.window > 0 ? fmin(hi, rows + a.window) : hi;
+  };
+  double least;
+  {  // fa_fwd.hip
+    const double n = ceil_div(a.N, 64), stage = W > 128 ? 64 : 128;
+    const bool pairs = a.causal && n > 1;
+    const double wgs = (pairs ? ceil_div(n, 2) : n) * BH;
+    const double first = ceil_div(keys(64, 64), stage), last = ceil_div(keys(64, 64 * n), stage);
+    const double steps = 0.5 * (first + last) * n * BH / wgs, tiles = pairs ? 2 : 1;
+    const FwdTimes& t = kTilesTimes[wi];
+    const bool masked = a.N % 64 || a.kv_len || a.window > 0 || a.alibi || a.seg_start || NK != a.N;
+    least = 1 + (kTilesW4[wi] > 0 && wgs >= 2 * kCUs && !(a.causal && masked)
+                     ? wgs / (2 * kCUs) * (steps * kTilesW4[wi] + tiles * t.ends)
+                     : equal_time(t, wgs, steps, tiles));
+  }
+  // A launch's work-items and the row blocks' indices stay within 32 bits.
+  constexpr double kMostItems = 4294967295.0;
+  auto consider = [&](FwdPlan p, double us) {
+    if (us >= least) return;
+    least = us;
+    best = p;
+  };
+  // What parts cost: a second launch (3 us, and 2 on the host, which small calls
+  // wait for) and the partial results to write and combine.
+  auto merge = [&](double items, int parts) {
+    return parts == 1 ? 0.0 : 5.0 + 0.0137 * items * parts * W / 128;
+  };
+  const bool split = NK > a.N && !a.seg_start;  // square calls' results do not depend on a workspace
+  constexpr int kTried[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+  if (!a.alibi) {  // fa_rows.hip
+    for (const int waves : {4, 8}) {
+      const double rows = 32.0 * waves, n = ceil_div(a.N, rows);
+      const double first = ceil_div(keys(rows, rows), 64), last = ceil_div(keys(rows, rows * n), 64);
+      const double total = 0.5 * (first + last) * n * BH, items = n * waves * BH;
+      const FwdTimes& t = waves == 4 ? kRows4Times[wi] : kRows8Times[wi];
+      if (n * BH * 512 > kMostItems) continue;
+      for (const int parts : kTried) {
+        if (parts > 16 || (parts > 1 && (!split || last < 2 * parts || items * parts > 8192))) break;
+        const double us = a.causal && n > 1 ? uneven_time(t, n * BH * parts, total, last / parts)
+                                            : equal_time(t, n * BH * parts, ceil(last / parts), 1);
+        consider({FwdPlan::kRows, waves, false, parts, (int)(n * waves), (int)items},
+                 us + merge(items, parts));
+      }
+      if (waves == 4 && a.causal && n > 1) {
+        const double wgs = ceil_div(n, 2) * BH;
+        consider({FwdPlan::kRows, 4, true, 1, (int)(n * waves), (int)items},
+                 equal_time(kPairTimes[wi], wgs, total / wgs, 2));
+      }
     }
   }
-  const double q_tiles = (a.N + 63) / 64, per_wg = a.causal && q_tiles > 1 ? 2 : 1;
-  const double wgs = ceil(q_tiles / per_wg) * a.B * a.Hq;
-  const double there = ceil(wgs / kCUs) * per_wg * (seen / (W > 128 ? 64 : 128) + 2.0);
-  return least < there ? DecPlan{(int)tiles, (int)items, best} : none;
+  if (split) {  // fa_dec.hip
+    const double tiles = ceil_div((double)(a.Hq / a.Hkv) * a.N, 32), items = tiles * a.B * a.Hkv;
+    const double seen = keys(a.N, a.N), read = 4.0 * a.B * a.Hkv * seen * a.D / 6.3e6;
+    if (items * (W / 32) * 512 <= kMostItems) {
+      for (const int parts : kTried) {
+        if (parts > 1 && (seen < 128.0 * parts || items * parts > 8192)) break;
+        const double rounds = ceil_div(ceil_div(seen, parts), W > 128 ? 128 : 256) * kDecTimes[wi];
+        const double n = items * parts, full = floor(n / kCUs), rest = n - full * kCUs;
+        double us = full * (rounds * 1.36 + 1.3);
+        if (rest > 0) us += rounds * (rest < kCUs / 2 ? 1.0 : 1.36) + 1.3;
+        consider({FwdPlan::kDec, 0, false, parts, (int)tiles, (int)items},
+                 2 + fmax(us, read) + merge(items, parts));
+      }
+    }
+  }
+  return best;
 }
 
 hipError_t launch_fwd(const FwdArgs& a, void* workspace) {
-  DecPlan plan = dec_plan(a);
-  if (plan.items > 0) {
-    if (!workspace) plan.parts = 1;
-    return by_width(a, a.dtype == kBF16, [&](auto w, auto bf, const FwdArgs& a) {
-      return launch_dec_w<decltype(w)::value, decltype(bf)::value>(a, plan, workspace);
-    });
-  }
-  return by_width(a, a.dtype == kBF16, [](auto w, auto bf, const FwdArgs& a) {
-    return launch_fwd_w<decltype(w)::value, decltype(bf)::value>(a);
+  FwdPlan plan = fwd_plan(a);
+  if (!workspace) plan.parts = 1;
+  const bool bf = a.dtype == kBF16;
+  const hipError_t e = by_width(a, bf, [&](auto w, auto bf, const FwdArgs& a) {
+    constexpr int W = decltype(w)::value;
+    constexpr bool BF = decltype(bf)::value;
+    switch (plan.kind) {
+      case FwdPlan::kRows: return launch_rows_w<W, BF>(a, plan, workspace);
+      case FwdPlan::kDec: return launch_dec_w<W, BF>(a, plan, workspace);
+      default: return launch_fwd_w<W, BF>(a);
+    }
+  });
+  if (e != hipSuccess || plan.parts <= 1) return e;
+  return by_width(a, bf, [&](auto w, auto bf, const FwdArgs& a) {
+    return launch_merge_w<decltype(w)::value, decltype(bf)::value>(a, plan, workspace);
   });
 }
 
