@@ -246,6 +246,11 @@ hipError_t launch_dropout_bits(uint64_t seed, uint32_t threshold, int P, int N, 
 hipError_t launch_pack_blocks(const uint8_t* layout, int Bl, int Hl, int B, int Hq, int Hkv,
                               int nb, bool causal, int* rows, int* cols, void* stream);
 
+// Bounds of packed sequences: rows of N ids (int32, or int64 when `wide`) at
+// the given element strides to dense (B, N) start and end (FwdArgs::seg_start).
+hipError_t launch_segment_bounds(const void* ids, bool wide, int B, int N, long long stride_b,
+                                 long long stride_n, int* start, int* end, void* stream);
+
 // Work-items (workgroups x threads) of the largest launch each pass makes for
 // a shape (either masking). An AMD dispatch packet counts its grid in
 // work-items in 32-bit fields, and the kernels number their work items with

@@ -508,6 +508,22 @@ std::vector<at::Tensor> fa_pack_blocks_t(at::Tensor layout, int64_t B, int64_t H
   return {rows, cols};
 }
 
+// (seg_start, seg_end) of packed sequences (fa_segment_bounds).
+std::vector<at::Tensor> fa_segment_bounds_t(at::Tensor ids) {
+  TORCH_CHECK(ids.is_cuda() && ids.dim() == 2, "segment ids must be a CUDA tensor (B, N)");
+  const bool wide = ids.scalar_type() == at::kLong;
+  TORCH_CHECK(wide || ids.scalar_type() == at::kInt, "segment ids must be int32 or int64");
+  c10::DeviceGuard guard(ids.device());
+  auto opts = ids.options().dtype(at::kInt);
+  auto start = at::empty({ids.size(0), ids.size(1)}, opts);
+  auto end = at::empty({ids.size(0), ids.size(1)}, opts);
+  check_rc(fa_segment_bounds(ids.data_ptr(), wide ? 1 : 0, (int)ids.size(0), (int)ids.size(1),
+                             ids.stride(0), ids.stride(1), start.data_ptr<int>(),
+                             end.data_ptr<int>(), current_stream(ids)),
+           "fa_segment_bounds");
+  return {start, end};
+}
+
 // Dense boolean mask (..., N, N) (nonzero = may attend) to the packed words
 // the kernels read: bits (..., N, ceil(N/32)) and, with `transposed`, bits_t
 // of the same shape holding the transpose (see fa_pack_mask).
@@ -576,6 +592,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "block-sparse layout (B|1, Hq|1, nb, nb) to the kernels' block lists",
         py::arg("layout"), py::arg("B"), py::arg("Hq"), py::arg("Hkv"), py::arg("N"),
         py::arg("causal"));
+  m.def("segment_bounds", &fa_segment_bounds_t,
+        "Bounds (seg_start, seg_end) of packed sequences from (B, N) ids", py::arg("ids"));
   m.def("pack_mask", &fa_pack_mask_t,
         "Bit-packs a dense boolean (..., N, N) mask for the mask / mask_t arguments",
         py::arg("mask"), py::arg("transposed") = true);

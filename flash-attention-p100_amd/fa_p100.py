@@ -431,11 +431,17 @@ def segment_bounds(segment_ids):
 
     A sequence is a maximal run of equal ids along a row: token i belongs to
     the run [seg_start[b, i], seg_end[b, i]). These are the bounds the kernels
-    take (fa_options.seg_start / seg_end in the C ABI). Computed with a few
-    device-side scans; nothing is copied to the host.
+    take (fa_options.seg_start / seg_end in the C ABI). One HIP kernel for int32
+    and int64 ids on the GPU, device-side torch scans for any others; nothing is
+    copied to the host.
     """
     s = segment_ids
     B, N = s.shape
+    # (subclasses and functorch's wrapped tensors have no storage of their own)
+    if s.is_cuda and s.dtype in (torch.int32, torch.int64) and 0 < B < 1 << 23 \
+            and 0 < N < (1 << 31) - (1 << 16) and type(s) is torch.Tensor \
+            and not torch._C._functorch.is_functorch_wrapped_tensor(s):
+        return tuple(_ext.segment_bounds(s))
     idx = torch.arange(N, device=s.device, dtype=torch.int64).expand(B, N)
     change = s[:, 1:] != s[:, :-1]  # a new run starts at i + 1
     starts = torch.ones(B, N, dtype=torch.bool, device=s.device)

@@ -358,6 +358,16 @@ int fa_pack_mask(const uint8_t* dense, int P, int N, uint32_t* bits, uint32_t* b
 int fa_dropout_bits(uint64_t seed, float p, int P, int N, uint32_t* bits, uint32_t* bits_t,
                     void* stream);
 /*
+ * Bounds of packed sequences for fa_options.seg_start / seg_end: a sequence is
+ * a maximal run of equal ids along one of B rows of N ids, int32 or (wide
+ * nonzero) int64, at element strides stride_b and stride_n; token i of row b
+ * belongs to the run [seg_start[b * N + i], seg_end[b * N + i]). No counterpart
+ * in the reference.
+ */
+int fa_segment_bounds(const void* ids, int wide, int B, int N, long long stride_b,
+                      long long stride_n, int* seg_start, int* seg_end, void* stream);
+
+/*
  * fa_dropout_bits for causal attention with as many key rows as query rows:
  * the same draw with every bit of a key j > i (row i) cleared, in both
  * layouts. Causal masking never reads those bits, so attention results are
