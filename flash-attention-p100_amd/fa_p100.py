@@ -50,6 +50,7 @@ _ext = _load_ext()
 
 # Rows and keys per block of a block-sparse layout (flash_attn's block_mask).
 BLOCK_SIZE = 128
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _bnhd_storage(t):
@@ -343,6 +344,16 @@ def flash_attn(q, k, v, causal=False, full_precision=False, kv_len=None, sliding
                                  f"{[tuple(t.shape) for t in blocks]}")
         else:
             blocks = pack_blocks(block_mask, q.size(0), q.size(1), k.size(1), q.size(2), causal)
+    # Calls without these inputs take the same Function in C++ (no interpreter
+    # between the launches); functorch transforms, tracing and tensor subclasses
+    # stay with the Python one, which they know how to handle or refuse.
+    if mask is None and drop is None and bias is None and blocks is None \
+            and type(q) in _PLAIN and type(k) in _PLAIN and type(v) in _PLAIN \
+            and torch._C._functorch.peek_interpreter_stack() is None \
+            and not torch.compiler.is_compiling():
+        start, end = segs if segs is not None else (None, None)
+        return _ext.flash_attn(q, k, v, causal, full_precision, kv_len, window, alibi_slopes,
+                               start, end, scale)
     return _FlashAttnP100.apply(q, k, v, causal, full_precision, kv_len, window, alibi_slopes,
                                 segs, scale, mask, drop, bias, blocks)
 
