@@ -141,8 +141,8 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(const half_t* __restrict__
                                                       const half_t* __restrict__ dO,
                                                       const float* __restrict__ Lse,
                                                       float* __restrict__ dvec,
-                                                      float* __restrict__ lse2, long rows,
-                                                      int Hq, int N, Strides st,
+                                                      float* __restrict__ lse2, unsigned rows,
+                                                      int Hq, int N, bool bnhd, Strides st,
                                                       unsigned* __restrict__ counters,
                                                       int n_counters, int dr) {
   constexpr int kLanesPerRow = pre_lanes_per_row(D);
@@ -151,13 +151,28 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(const half_t* __restrict__
   // The main kernel's split-tile counters start at zero (it leaves them zero,
   // but a fresh workspace holds anything). n_counters < rows <= threads.
   if (const long c = (long)blockIdx.x * 256 + tid; c < n_counters) counters[c] = 0u;
-  const long row = (long)blockIdx.x * kRowsPerBlock + tid / kLanesPerRow;
+  // Rows in the order in which they lie in memory, (b, h, n) or (b, n, h), so
+  // that consecutive workgroups read consecutive bytes; rows x lanes fits 32
+  // bits (the launch's work-items). With 64-bit divisions and (b, h, n) order
+  // for both layouts the (B, N, H, D) pass at B=1 H=16 N=8192 D=128 took 21 us.
+  const unsigned r = blockIdx.x * (unsigned)kRowsPerBlock + tid / kLanesPerRow;
+  unsigned b, hq, n;
+  if (bnhd) {
+    const unsigned bn = r / Hq;
+    hq = r - bn * Hq;
+    b = bn / N;
+    n = bn - b * N;
+  } else {
+    const unsigned bh = r / N;
+    n = r - bh * N;
+    b = bh / Hq;
+    hq = bh - b * Hq;
+  }
+  const size_t row = ((size_t)b * Hq + hq) * N + n;  // of the dense (B, Hq, N) vectors
   const int c8 = (tid % kLanesPerRow) * 8;
   float acc = 0.f;
-  if (row < rows && c8 < dr) {
-    // row = (b * Hq + hq) * N + n over the dense (B, Hq, N) vectors.
-    const long bh = row / N, n = row - bh * N;
-    const size_t off = (size_t)((bh / Hq) * st.b + (bh % Hq) * st.h + n * st.n) + c8;
+  if (r < rows && c8 < dr) {
+    const size_t off = (size_t)(b * st.b + hq * st.h) + (size_t)n * st.n + c8;
     const half8 o = as_half8(*reinterpret_cast<const u32x4*>(O + off));
     const half8 g = as_half8(*reinterpret_cast<const u32x4*>(dO + off));
 #pragma unroll
@@ -165,7 +180,7 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(const half_t* __restrict__
   }
 #pragma unroll
   for (int off = kLanesPerRow / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-  if (row < rows && (tid % kLanesPerRow) == 0) {
+  if (r < rows && (tid % kLanesPerRow) == 0) {
     dvec[row] = acc;
     lse2[row] = Lse[row] * kLog2e;
   }
@@ -1139,8 +1154,8 @@ hipError_t launch_pre_d(const BwdArgs& a) {
   const long rows = (long)a.B * a.Hq * a.N;
   const dim3 grid((unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock));
   hipLaunchKernelGGL((bwd_pre_kernel<D, BF>), grid, dim3(256), 0, (hipStream_t)a.stream,
-                     (const half_t*)a.o, (const half_t*)a.dO, a.lse, a.dvec, a.lse2, rows, a.Hq,
-                     a.N, make_strides(a.layout, a.Hq, a.N, a.D), a.counters, a.n_counters, a.D);
+                     (const half_t*)a.o, (const half_t*)a.dO, a.lse, a.dvec, a.lse2,
+                     (unsigned)rows, a.Hq, a.N, a.layout == kBNHD, make_strides(a.layout, a.Hq, a.N, a.D), a.counters, a.n_counters, a.D);
   return hipGetLastError();
 }
 

@@ -210,7 +210,13 @@ double ceil_div(double a, double b) { return ceil(a / b); }
 
 FwdPlan fwd_plan(const FwdArgs& a) {
   FwdPlan best{FwdPlan::kTiles, 0, false, 1, 0, 0};
-  if (a.mask || a.drop || a.bias || a.block_rows) return best;
+  // fa_rows.hip takes dropout or a bias alone (its bias rows load 16 bytes at a
+  // time), at widths up to 128; the other per-score inputs stay on fa_fwd.hip.
+  const bool feat = a.drop || a.bias;
+  if (a.mask || a.block_rows || (a.drop && a.bias) || (feat && a.D > 128)) return best;
+  if (a.bias && ((a.N | a.bias_sb | a.bias_sh) % 4 != 0 ||
+                 (reinterpret_cast<uintptr_t>(a.bias) & 15) != 0))
+    return best;
   const int NK = key_rows(a.N, a.Nkv), W = padded_head_dim(a.D);
   const int wi = W <= 32 ? kW32 : W <= 64 ? kW64 : W <= 96 ? kW96 : W <= 128 ? kW128 : kW256;
   const double BH = (double)a.B * a.Hq, kofs = NK - a.N;
@@ -232,6 +238,14 @@ FwdPlan fwd_plan(const FwdArgs& a) {
                      ? wgs / (2 * kCUs) * (steps * kTilesW4[wi] + tiles * t.ends)
                      : equal_time(t, wgs, steps, tiles));
   }
+  // These inputs cost the two kernels differently: a bias takes fa_fwd.hip 2.6
+  // times as long as none and fa_rows.hip 1.6 times (B=4 H=8 N=1024 D=64 dense:
+  // 51 -> 28 us, B=1 H=16 N=4096 D=64 causal: 217 -> 136, B=2 H=32 N=1500 D=128
+  // causal: 185 -> 125); dropout costs fa_rows.hip more than fa_fwd.hip's unmasked
+  // copies (79 us there and 82 here at B=1 H=16 N=4096 D=64 causal) and as much as
+  // its masked ones, which a ragged N takes (96 -> 72 us at B=2 H=32 N=1500 D=128).
+  if (a.bias) least *= 1.6;
+  if (a.drop && a.N % 128 == 0) least *= 0.85;
   // A launch's work-items and the row blocks' indices stay within 32 bits.
   constexpr double kMostItems = 4294967295.0;
   auto consider = [&](FwdPlan p, double us) {
@@ -248,6 +262,7 @@ FwdPlan fwd_plan(const FwdArgs& a) {
   constexpr int kTried[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   if (!a.alibi) {  // fa_rows.hip
     for (const int waves : {4, 8}) {
+      if (feat && waves == 8) continue;
       const double rows = 32.0 * waves, n = ceil_div(a.N, rows);
       const double first = ceil_div(keys(rows, rows), 64), last = ceil_div(keys(rows, rows * n), 64);
       const double total = 0.5 * (first + last) * n * BH, items = n * waves * BH;

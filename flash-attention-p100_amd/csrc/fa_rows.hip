@@ -19,6 +19,12 @@
 // bottom right, windows, key lengths and packed sequences all come down to
 // these bounds, of which neither decreases with i; only the stages at the ends
 // of a wave's bounds test them, and stages outside them are skipped.
+//
+// Dropout (FEAT kFeatDrop): a lane's keep bits of the next stage (two words of
+// its row) load during this one. Bias (kFeatBias): each wave's 32 x 64 values of
+// the next stage load into LDS of its own as soon as this stage's are in the
+// score accumulators, which they initialise (fa_fwd.hip reads them per lane
+// from rows N floats apart, 32 cache lines per load).
 #include <type_traits>
 
 #include "fa_device.h"
@@ -53,6 +59,11 @@ struct RowsArgs {
   float2* part_ml;  // (parts > 1; DecArgs' layout)
   int N, NK, Hq, group, n_tiles, BH, parts, causal, window, dr;
   float scale_log2;
+  const uint32_t* drop;  // as FwdArgs (kFeatDrop, kFeatBias instantiations)
+  float drop_scale;
+  const float* bias;
+  long long bias_sb, bias_sh;
+  float bias_raw;  // 1 / softmax scale
   const int* kv_len;
   const int* seg_start;
   const int* seg_end;
@@ -61,7 +72,7 @@ struct RowsArgs {
 
 // PAIR (causal): a workgroup takes query tile T-1-x, then x, so that all do the
 // same work; without it the tiles start longest first.
-template <int D, int NW, bool PAIR, bool BF>
+template <int D, int NW, bool PAIR, int FEAT, bool BF>
 __global__ __launch_bounds__((Rows<D, NW>::kThreads)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void rows_kernel(const RowsArgs a) {
   using R = Rows<D, NW>;
@@ -72,6 +83,10 @@ void rows_kernel(const RowsArgs a) {
   __shared__ __align__(16) half_t vt0[R::kTileHalves];
   __shared__ __align__(16) half_t kt1[R::kTileHalves];
   __shared__ __align__(16) half_t vt1[R::kTileHalves];
+  constexpr bool DROP = FEAT == kFeatDrop, BIAS = FEAT == kFeatBias;
+  // Bias rows of a wave: 64 floats, 16-byte chunk c of row r at position c ^
+  // (r % 16), so that 16 rows' reads of one chunk hit 16 bank groups.
+  __shared__ __align__(16) float bt[BIAS ? NW * 32 * kKeys : 4];
   const int gx = PAIR ? (a.n_tiles + 1) / 2 : a.n_tiles;
   const int w = xcd_work_index(gx * a.parts * a.BH);
   if (w < 0) return;
@@ -136,6 +151,25 @@ void rows_kernel(const RowsArgs a) {
     for (int cb = 0; cb < D / 32; ++cb) oacc[cb] = zero16();
     float m_raw = -INFINITY, l = 0.f;
     if (PAIR && turn) __syncthreads();  // the last tile's stages have been read
+    const int W32 = (a.N + 31) >> 5;
+    const uint32_t* zrow =
+        DROP ? a.drop + ((size_t)bh * a.N + min(i_row, a.N - 1)) * W32 : nullptr;
+    auto zword = [&](int j, int t) { return DROP ? zrow[min(2 * j + t, W32 - 1)] : ~0u; };
+    uint32_t zw[2] = {zword(first, 0), zword(first, 1)};
+    const rsrc_t rb = bias_rows_rsrc(BIAS ? a.bias + b * a.bias_sb + hq * a.bias_sh : nullptr,
+                                     i_base, a.N);
+    // Instruction u covers the wave's rows 4u .. 4u+3.
+    auto bload = [&](int j) {
+      if constexpr (BIAS) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int r = 4 * u + (lane >> 4);
+          lds_direct_buf<16>(bt, rb, (uint32_t)(r * a.N) * 4u + ((lane ^ r) & 15) * 16u,
+                             (uint32_t)(j * kKeys) * 4u, (uint32_t)(wave * 32 * kKeys + u * 256) * 4u);
+        }
+      }
+    };
+    bload(first);
 #pragma unroll
     for (int u = 0; u < kParts; ++u) {
       plan.part(kt0, rk, first * kKeys, wave, u);
@@ -156,15 +190,38 @@ void rows_kernel(const RowsArgs a) {
         }
       };
       const int base = j * kKeys;
+      const uint32_t zc[2] = {zw[0], zw[1]};
+      if constexpr (DROP) {
+        zw[0] = zword(min(j + 1, last - 1), 0);
+        zw[1] = zword(min(j + 1, last - 1), 1);
+      }
       if (none || base >= w_hi || base + kKeys <= w_lo) {  // no key for any row of the wave
 #pragma unroll
         for (int u = 0; u < 2 * kParts; ++u) issue(u);
+        if constexpr (BIAS) bload(min(j + 1, last - 1));
         return;
       }
       floatx16 s[2];
+      if constexpr (BIAS) {
+        const float* brow = bt + wave * 32 * kKeys + l32 * kKeys;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const floatx4 x =
+                *reinterpret_cast<const floatx4*>(brow + (((8 * t + 2 * g + h) ^ l32) & 15) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[t][4 * g + e] = x[e] * a.bias_raw;
+          }
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // the reads are done before the loads below
+        __builtin_amdgcn_sched_barrier(0);
+        bload(min(j + 1, last - 1));
+      } else {
+        s[0] = zero16();
+        s[1] = zero16();
+      }
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        s[t] = zero16();
 #pragma unroll
         for (int kk = 0; kk < D / 16; ++kk) {
           s[t] = mfma16<BF>(tile_read16<D>(Ks, 32 * t, kk, roff), qb[kk], s[t]);
@@ -207,7 +264,9 @@ void rows_kernel(const RowsArgs a) {
         for (int e = 0; e < 16; ++e) {
           const float p = fast_exp2(fmaf(s[t][e], c, neg));
           l += p;
-          pb[2 * t + (e >> 3)][e & 7] = to16<BF>(p);
+          // Dropout: the row sum keeps every key, P V only the kept ones.
+          const bool keep = !DROP || ((zc[t] >> (4 * h)) >> (8 * (e >> 2) + (e & 3))) & 1u;
+          pb[2 * t + (e >> 3)][e & 7] = to16<BF>(keep ? p : 0.f);
         }
 #pragma unroll
       for (int q = 0; q < 4; ++q)
@@ -234,7 +293,8 @@ void rows_kernel(const RowsArgs a) {
               floatx4{oacc[cb][4 * g], oacc[cb][4 * g + 1], oacc[cb][4 * g + 2], oacc[cb][4 * g + 3]};
       if (h == 0) a.part_ml[slot * 32 + l32] = make_float2(m_raw * c, l_all);
     } else if (i_row < a.N) {
-      const float inv_l = l_all > 0.f ? 1.f / l_all : 0.f;  // a row without keys: O = 0
+      // (a row without keys: O = 0; dropout scales the kept keys)
+      const float inv_l = l_all > 0.f ? (DROP ? a.drop_scale : 1.f) / l_all : 0.f;
       half_t* orow = a.o + b * a.stq.b + hq * a.stq.h + (size_t)i_row * a.stq.n;
 #pragma unroll
       for (int cb = 0; cb < D / 32; ++cb)
@@ -253,10 +313,10 @@ void rows_kernel(const RowsArgs a) {
   }
 }
 
-template <int D, int NW, bool PAIR, bool BF>
+template <int D, int NW, bool PAIR, int FEAT, bool BF>
 hipError_t launch_rows_t(const RowsArgs& a, hipStream_t stream) {
   const int gx = PAIR ? (a.n_tiles + 1) / 2 : a.n_tiles;
-  hipLaunchKernelGGL((rows_kernel<D, NW, PAIR, BF>),
+  hipLaunchKernelGGL((rows_kernel<D, NW, PAIR, FEAT, BF>),
                      dim3((unsigned)xcd_grid(gx * a.parts * a.BH)), dim3(Rows<D, NW>::kThreads), 0,
                      stream, a);
   return hipGetLastError();
@@ -294,9 +354,23 @@ hipError_t launch_rows_w<FA_WIDTH, FA_BF>(const FwdArgs& a, const FwdPlan& plan,
     d.part_o = (float*)((char*)workspace + part_ml_bytes(plan));
   }
   const hipStream_t stream = (hipStream_t)a.stream;
-  if (plan.waves == 8) return launch_rows_t<D, 8, false, FA_BF>(d, stream);
-  return plan.pair ? launch_rows_t<D, 4, true, FA_BF>(d, stream)
-                   : launch_rows_t<D, 4, false, FA_BF>(d, stream);
+  d.drop = a.drop;
+  d.drop_scale = a.drop_scale;
+  d.bias = a.bias;
+  d.bias_sb = a.bias_sb;
+  d.bias_sh = a.bias_sh;
+  d.bias_raw = 1.f / (a.scale > 0.f ? a.scale : 1.f / sqrtf((float)a.D));
+  if constexpr (D <= 128) {  // (the plan keeps width 256 with these inputs on fa_fwd.hip)
+    if (a.drop)
+      return plan.pair ? launch_rows_t<D, 4, true, kFeatDrop, FA_BF>(d, stream)
+                       : launch_rows_t<D, 4, false, kFeatDrop, FA_BF>(d, stream);
+    if (a.bias)
+      return plan.pair ? launch_rows_t<D, 4, true, kFeatBias, FA_BF>(d, stream)
+                       : launch_rows_t<D, 4, false, kFeatBias, FA_BF>(d, stream);
+  }
+  if (plan.waves == 8) return launch_rows_t<D, 8, false, 0, FA_BF>(d, stream);
+  return plan.pair ? launch_rows_t<D, 4, true, 0, FA_BF>(d, stream)
+                   : launch_rows_t<D, 4, false, 0, FA_BF>(d, stream);
 }
 
 }  // namespace fa

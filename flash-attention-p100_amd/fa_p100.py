@@ -132,7 +132,11 @@ class _FlashAttnP100(torch.autograd.Function):
         dbias = None
         if ctx.bias is not None and ctx.needs_input_grad[12]:  # bias is input 12
             B, H, N = grad_o.size(0), grad_o.size(1), grad_o.size(2)
-            dbias = torch.zeros(B, H, N, N, dtype=torch.float32, device=grad_o.device)
+            # The kernel writes the pairs of query blocks and keys it steps over:
+            # all of them, unless something bounds a row's keys.
+            whole = not (ctx.causal or ctx.kv_len is not None or ctx.segs is not None)
+            dbias = (torch.empty if whole else torch.zeros)(
+                B, H, N, N, dtype=torch.float32, device=grad_o.device)
         if ctx.bnhd:
             qb, kb, vb, ob, lse = ctx.saved_tensors
             gb = grad_o.transpose(1, 2).contiguous()

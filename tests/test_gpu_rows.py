@@ -87,3 +87,79 @@ def test_rows_bounds(option, causal):
     o, lse = fa_p100._ext.forward_dt(*(t.to(DEV) for t in (q, k, v)), causal, **kw)
     for b in range(B):
         check(o, lse, q, k, v, causal, b, Hq - 1, **okw[b])
+
+
+FEAT_CASES = [
+    # B, H, N, D, causal: N a multiple of 4 (the bias rows' 16-byte loads), ragged
+    # against stages of 64 keys and tiles of 128 rows
+    (4, 8, 300, 64, False),
+    (8, 12, 516, 64, True),
+    (3, 16, 260, 96, True),
+    (2, 32, 388, 128, True),
+    (12, 8, 132, 32, False),
+    (4, 16, 1284, 64, True),  # paired tiles
+]
+
+
+@pytest.mark.parametrize("feature", ["bias", "bias_shared", "dropout", "kv_len"])
+@pytest.mark.parametrize("B,H,N,D,causal", FEAT_CASES)
+def test_rows_bias_and_dropout(B, H, N, D, causal, feature):
+    """A bias per head and one shared by all (rows of one plane through every
+    head's loads), -inf and the type's lowest value in it, dropout's keep bits,
+    and a bias with key lengths."""
+    import fa_p100
+    q, k, v = make(B, H, H, N, N, D, seed=N)
+    dev = [t.to(DEV) for t in (q, k, v)]
+    g = torch.Generator().manual_seed(1)
+    slices = ((0, 0), (B - 1, H - 1))
+    if feature == "dropout":
+        z, _, zs = fa_p100.dropout_bits(77, 0.2, B, H, N, DEV, causal=causal)
+        o, lse = fa_p100._ext.forward_dt(*dev, causal, drop=z, drop_scale=zs)
+        for b, h in slices:
+            words = z[b, h].cpu().numpy().view(np.uint32)
+            keep = ((words[:, :, None] >> np.arange(32, dtype=np.uint32)) & 1).astype(bool)
+            keep = keep.reshape(N, -1)[None, None, :, :N]
+            # (P / (1 - p): the bar scales with it)
+            check_drop(o, lse, q, k, v, causal, b, h, (keep, zs))
+        return
+    shape = (1, 1, N, N) if feature == "bias_shared" else (1, H, N, N)
+    bias = torch.randn(shape, generator=g)
+    bias[..., 3::7] = -float("inf")  # hidden keys
+    bias[..., 1, :] = torch.finfo(torch.float32).min  # a row of the lowest value
+    bias[..., 1, 0] = 0.0
+    kw, lens = {}, [N] * B
+    if feature == "kv_len":
+        lens = [max(1, N - 37 * b) for b in range(B)]
+        kw["kv_len"] = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    o, lse = fa_p100._ext.forward_dt(*dev, causal, bias=bias.to(DEV), **kw)
+    for b, h in slices:
+        plane = bias[:, h:h + 1] if shape[1] > 1 else bias
+        check(o, lse, q, k, v, causal, b, h, bias=np64(plane), kv_len=[lens[b]])
+
+
+def check_drop(o, lse, q, k, v, causal, b, h, dropout):
+    args = [np64(t[b:b + 1, h:h + 1]) for t in (q, k, v)]
+    ref_o, ref_lse = ora.attention_fwd(*args, causal, dropout=dropout)
+    assert ora.max_abs(np64(o[b:b + 1, h:h + 1]), ref_o) <= FWD_MAX_ABS * dropout[1] ** 2
+    assert ora.max_abs(np64(lse[b:b + 1, h:h + 1]), ref_lse) <= LSE_MAX_ABS
+
+
+def test_bias_gradient_is_written_whole():
+    """Without causal masking, lengths or sequences the backward writes every
+    element of the bias's gradient, into memory that held NaN."""
+    import fa_p100
+    for N in (130, 256):
+        q, k, v, do = (torch.randn(2, 4, N, 64, device=DEV).half() for _ in range(4))
+        bias = torch.randn(1, 4, N, N, device=DEV, requires_grad=True)
+        junk = torch.full((2, 4, N, N), float("nan"), device=DEV)
+        torch.cuda.synchronize()
+        del junk  # its block serves the gradient
+        o = fa_p100.flash_attn(q, k, v, attn_bias=bias)
+        (db,) = torch.autograd.grad(o, bias, do)
+        assert torch.isfinite(db).all()
+        s = (q.float() @ k.float().transpose(-1, -2).contiguous() / 8 + bias.detach())
+        p = s.softmax(-1)
+        dp = do.float() @ v.float().transpose(-1, -2).contiguous()
+        ds = p * (dp - (dp * p).sum(-1, keepdim=True))
+        ref = ds.sum(0, keepdim=True)
+        assert ((db - ref).norm() / ref.norm()).item() <= 5e-3
