@@ -210,10 +210,12 @@ double ceil_div(double a, double b) { return ceil(a / b); }
 
 FwdPlan fwd_plan(const FwdArgs& a) {
   FwdPlan best{FwdPlan::kTiles, 0, false, 1, 0, 0};
-  // fa_rows.hip takes dropout or a bias alone (its bias rows load 16 bytes at a
-  // time), at widths up to 128; the other per-score inputs stay on fa_fwd.hip.
-  const bool feat = a.drop || a.bias;
-  if (a.mask || a.block_rows || (a.drop && a.bias) || (feat && a.D > 128)) return best;
+  // fa_rows.hip takes dropout, a bias (whose rows load 16 bytes at a time) or
+  // ALiBi alone, the first two at widths up to 128; the other per-score inputs
+  // stay on fa_fwd.hip.
+  const bool feat = a.drop || a.bias || a.alibi;
+  if (a.mask || a.block_rows || (a.drop && a.bias) || ((a.drop || a.bias) && (a.alibi || a.D > 128)))
+    return best;
   if (a.bias && ((a.N | a.bias_sb | a.bias_sh) % 4 != 0 ||
                  (reinterpret_cast<uintptr_t>(a.bias) & 15) != 0))
     return best;
@@ -260,7 +262,7 @@ FwdPlan fwd_plan(const FwdArgs& a) {
   };
   const bool split = NK > a.N && !a.seg_start;  // square calls' results do not depend on a workspace
   constexpr int kTried[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
-  if (!a.alibi) {  // fa_rows.hip
+  {  // fa_rows.hip
     for (const int waves : {4, 8}) {
       if (feat && waves == 8) continue;
       const double rows = 32.0 * waves, n = ceil_div(a.N, rows);

@@ -33,6 +33,7 @@
 namespace fa {
 namespace {
 
+constexpr int kFeatAlibi = 64;  // (a FEAT bit beside Feat's)
 constexpr float kRescaleLog2 = 8.f;  // as the forward's lazy rescale
 
 template <int D, int NW>
@@ -61,6 +62,7 @@ struct RowsArgs {
   float scale_log2;
   const uint32_t* drop;  // as FwdArgs (kFeatDrop, kFeatBias instantiations)
   float drop_scale;
+  const float* alibi;  // (kFeatAlibi)
   const float* bias;
   long long bias_sb, bias_sh;
   float bias_raw;  // 1 / softmax scale
@@ -83,7 +85,7 @@ void rows_kernel(const RowsArgs a) {
   __shared__ __align__(16) half_t vt0[R::kTileHalves];
   __shared__ __align__(16) half_t kt1[R::kTileHalves];
   __shared__ __align__(16) half_t vt1[R::kTileHalves];
-  constexpr bool DROP = FEAT == kFeatDrop, BIAS = FEAT == kFeatBias;
+  constexpr bool DROP = FEAT == kFeatDrop, BIAS = FEAT == kFeatBias, ALIBI = FEAT == kFeatAlibi;
   // Bias rows of a wave: 64 floats, 16-byte chunk c of row r at position c ^
   // (r % 16), so that 16 rows' reads of one chunk hit 16 bank groups.
   __shared__ __align__(16) float bt[BIAS ? NW * 32 * kKeys : 4];
@@ -114,6 +116,8 @@ void rows_kernel(const RowsArgs a) {
   };
 
   const float c = a.scale_log2, thr_raw = kRescaleLog2 / c;
+  // ALiBi slope of this head in raw-score units.
+  const float slope = ALIBI ? a.alibi[hq] * kLog2e / c : 0.f;
   const int roff = row_lane_off<D>(lane), troff = tr_lane_off<D>(lane);
   const size_t kv_off = (size_t)(b * a.stk.b + hkv * a.stk.h);
   const rsrc_t rk = rows_rsrc(a.k + kv_off, a.NK, a.stk.n, a.dr);
@@ -230,6 +234,14 @@ void rows_kernel(const RowsArgs a) {
       }
 #pragma unroll
       for (int u = 2 * (D / 16); u < 2 * kParts; ++u) issue(u);
+      if constexpr (ALIBI) {  // -slope |i - j|, distances exact in fp32
+        const float d0 = (float)(i_row + kofs - base - 4 * h);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            s[t][e] = fmaf(-slope, fabsf(d0 - (float)(32 * t + 8 * (e >> 2) + (e & 3))), s[t][e]);
+      }
       if (base < all_lo || base + kKeys > all_hi) {
         const int d = base + 4 * h;
 #pragma unroll
@@ -360,7 +372,7 @@ hipError_t launch_rows_w<FA_WIDTH, FA_BF>(const FwdArgs& a, const FwdPlan& plan,
   d.bias_sb = a.bias_sb;
   d.bias_sh = a.bias_sh;
   d.bias_raw = 1.f / (a.scale > 0.f ? a.scale : 1.f / sqrtf((float)a.D));
-  if constexpr (D <= 128) {  // (the plan keeps width 256 with these inputs on fa_fwd.hip)
+  if constexpr (D <= 128) {  // (the plan keeps width 256 with these two on fa_fwd.hip)
     if (a.drop)
       return plan.pair ? launch_rows_t<D, 4, true, kFeatDrop, FA_BF>(d, stream)
                        : launch_rows_t<D, 4, false, kFeatDrop, FA_BF>(d, stream);
@@ -368,6 +380,10 @@ hipError_t launch_rows_w<FA_WIDTH, FA_BF>(const FwdArgs& a, const FwdPlan& plan,
       return plan.pair ? launch_rows_t<D, 4, true, kFeatBias, FA_BF>(d, stream)
                        : launch_rows_t<D, 4, false, kFeatBias, FA_BF>(d, stream);
   }
+  d.alibi = a.alibi;
+  if (a.alibi)
+    return plan.pair ? launch_rows_t<D, 4, true, kFeatAlibi, FA_BF>(d, stream)
+                     : launch_rows_t<D, 4, false, kFeatAlibi, FA_BF>(d, stream);
   if (plan.waves == 8) return launch_rows_t<D, 8, false, 0, FA_BF>(d, stream);
   return plan.pair ? launch_rows_t<D, 4, true, 0, FA_BF>(d, stream)
                    : launch_rows_t<D, 4, false, 0, FA_BF>(d, stream);

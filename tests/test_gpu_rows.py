@@ -163,3 +163,20 @@ def test_bias_gradient_is_written_whole():
         ds = p * (dp - (dp * p).sum(-1, keepdim=True))
         ref = ds.sum(0, keepdim=True)
         assert ((db - ref).norm() / ref.norm()).item() <= 5e-3
+
+
+@pytest.mark.parametrize("B,H,N,Nk,D,causal", [
+    (4, 8, 300, 300, 64, False),
+    (8, 12, 517, 517, 128, True),
+    (4, 16, 1285, 1285, 64, True),   # paired tiles
+    (3, 16, 261, 261, 256, True),
+    (1, 8, 1188, 5122, 96, True),    # distances from the last key's diagonal
+])
+def test_rows_alibi(B, H, N, Nk, D, causal):
+    import fa_p100
+    q, k, v = make(B, H, H, N, Nk, D, seed=N)
+    slopes = torch.tensor([2.0 ** (-8.0 * (h + 1) / H) for h in range(H)])
+    o, lse = fa_p100._ext.forward_dt(*(t.to(DEV) for t in (q, k, v)), causal,
+                                     alibi_slopes=slopes.to(DEV))
+    for b, h in ((0, 0), (B - 1, H - 1)):
+        check(o, lse, q, k, v, causal, b, h, alibi=slopes[h:h + 1].double().numpy())
