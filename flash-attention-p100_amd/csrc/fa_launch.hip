@@ -285,8 +285,11 @@ FwdPlan fwd_plan(const FwdArgs& a) {
     }
   }
   if (split) {  // fa_dec.hip
+    // (K and V come at 6 TB/s from 170 workgroups on, fewer cannot keep enough
+    // loads in flight: B=4 H=32/8 N=1, 32000 keys, D=128 takes 309, 173, 106 and
+    // 95 us with 1, 2, 4 and 8 parts of 32 workgroups)
     const double tiles = ceil_div((double)(a.Hq / a.Hkv) * a.N, 32), items = tiles * a.B * a.Hkv;
-    const double seen = keys(a.N, a.N), read = 4.0 * a.B * a.Hkv * seen * a.D / 6.3e6;
+    const double seen = keys(a.N, a.N), read = 4.0 * a.B * a.Hkv * seen * a.D / 6.0e6;
     if (items * (W / 32) * 512 <= kMostItems) {
       for (const int parts : kTried) {
         if (parts > 1 && (seen < 128.0 * parts || items * parts > 8192)) break;
@@ -295,7 +298,7 @@ FwdPlan fwd_plan(const FwdArgs& a) {
         double us = full * (rounds * 1.36 + 1.3);
         if (rest > 0) us += rounds * (rest < kCUs / 2 ? 1.0 : 1.36) + 1.3;
         consider({FwdPlan::kDec, 0, false, parts, (int)tiles, (int)items},
-                 2 + fmax(us, read) + merge(items, parts));
+                 2 + fmax(us, read * fmax(1.0, pow(170.0 / n, 0.6))) + merge(items, parts));
       }
     }
   }

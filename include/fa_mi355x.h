@@ -112,10 +112,12 @@ int fa_fwd_bnhd(const void* q, const void* k, const void* v, void* o, float* lse
 /*
  * Bytes of device workspace fa_bwd needs: two (B, Hq, N) float32 vectors, the
  * reference's `dvec` (fa_p100_ext.cu:124) and the saved LSE pre-multiplied by
- * log2(e); then B*Hq*floor(ceil(N/128)/2) uint32 counters; then, for each
- * (b, kv head) and each of those floor(ceil(N/128)/2) pairs of 128-row key
- * tiles, two fp32 partial-sum slots of 128*D*2 floats (the backward's causal
- * load balancing splits a short key tile's work between two workgroups).
+ * log2(e); then B*Hq*floor(ceil(N/128)/2) uint32 counters; then fp32
+ * partial-sum slots of 128*D*2 floats (D rounded up to 32, 64, 96, 128 or 256)
+ * for each (b, kv head): two for each of those floor(ceil(N/128)/2) pairs of
+ * 128-row key tiles (the backward's causal load balancing splits a key tile's
+ * work between two workgroups), or, where small grids share every key tile
+ * among up to 24 workgroups, one for each of them.
  * Each part is rounded up to 256 bytes. 0 for an invalid shape.
  */
 size_t fa_bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D);
