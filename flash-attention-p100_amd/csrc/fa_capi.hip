@@ -488,9 +488,9 @@ int fa_pack_blocks(const uint8_t* layout, int layout_b, int layout_h, int B, int
 int fa_segment_bounds(const void* ids, int wide, int B, int N, long long stride_b,
                       long long stride_n, int* seg_start, int* seg_end, void* stream) {
   if (N <= 0) return FA_ERR_SEQLEN;
-  // (one workgroup of 256 threads per row, token indices up to a tile past N)
+  // (one workgroup of 1024 threads per row, token indices up to a tile past N)
   if (B <= 0) return FA_ERR_BATCH;
-  if (B > (1 << 23) || N > INT_MAX - (1 << 16)) return FA_ERR_TOO_LARGE;
+  if (B > (1 << 21) || N > INT_MAX - (1 << 16)) return FA_ERR_TOO_LARGE;
   if (!ids || !seg_start || !seg_end) return FA_ERR_NULL;
   return to_code(fa::launch_segment_bounds(ids, wide != 0, B, N, stride_b, stride_n, seg_start,
                                            seg_end, stream));

@@ -305,10 +305,10 @@ unsigned blocks_for(long long items) {
 // of a run belongs to [start, end). One workgroup per row, kSegTile ids at a
 // time: a thread finds the run starts among its kSegPer consecutive ids, and a
 // scan over the threads carries the last start before them (forward, start[t])
-// or the next one after them (backward, end[t]). Latency-bound: 4 us at 4096
+// or the next one after them (backward, end[t]). Latency-bound: 7 us at 2 x 4096
 // ids, where the torch operators it replaces (comparisons, cummax, cummin and
 // flips over int64) were 15 launches of 94 us in all.
-constexpr int kSegThreads = 256, kSegPer = 16, kSegTile = kSegThreads * kSegPer;
+constexpr int kSegThreads = 1024, kSegPer = 4, kSegTile = kSegThreads * kSegPer;
 
 // Inclusive scan over the workgroup's threads, in thread order (forward) or
 // against it; `carry` comes before the first thread. Two barriers.

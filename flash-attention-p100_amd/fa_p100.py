@@ -453,7 +453,7 @@ def segment_bounds(segment_ids):
     s = segment_ids
     B, N = s.shape
     # (subclasses and functorch's wrapped tensors have no storage of their own)
-    if s.is_cuda and s.dtype in (torch.int32, torch.int64) and 0 < B < 1 << 23 \
+    if s.is_cuda and s.dtype in (torch.int32, torch.int64) and 0 < B <= 1 << 21 \
             and 0 < N < (1 << 31) - (1 << 16) and type(s) is torch.Tensor \
             and not torch._C._functorch.is_functorch_wrapped_tensor(s):
         return tuple(_ext.segment_bounds(s))
