@@ -13,7 +13,9 @@
 // the last four take bf16 as well as fp16; pack_mask bit-packs a boolean
 // mask for their `mask` / `mask_t` arguments and dropout_bits draws the keep
 // bits for `drop` / `drop_t`; they also take an fp32 attention `bias` (and
-// the backward its gradient buffer `dbias`).
+// the backward its gradient buffer `dbias`). segment_bounds finds packed
+// sequences' bounds, and flash_attn is the autograd Function over these entries
+// for the calls that need no packed mask, dropout, bias or block lists.
 //
 // Plain C++ (no device code): every launch goes through the C ABI of
 // libfa_mi355x.so (include/fa_mi355x.h). Unlike the reference, which uses the
