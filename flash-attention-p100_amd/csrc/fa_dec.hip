@@ -117,8 +117,10 @@ __global__ __launch_bounds__((Dec<D>::kThreads)) void dec_kernel(const DecArgs a
   const float alibi_raw = a.alibi ? a.alibi[hq] * kLog2e / c : 0.f;
   const int roff = row_lane_off<D>(lane), troff = tr_lane_off<D>(lane);
   const size_t kv_off = (size_t)(b * a.stk.b + hkv * a.stk.h);
-  const rsrc_t rk = rows_rsrc(a.k + kv_off, a.NK, a.stk.n, a.dr);
-  const rsrc_t rv = rows_rsrc(a.v + kv_off, a.NK, a.stk.n, a.dr);
+  // Rows from the key length on read as zeros: a masked key's P is zero, but
+  // zero times a NaN or an infinity that the padding holds would be NaN.
+  const rsrc_t rk = rows_rsrc(a.k + kv_off, Nk, a.stk.n, a.dr);
+  const rsrc_t rv = rows_rsrc(a.v + kv_off, Nk, a.stk.n, a.dr);
   TilePlan<D, kKeys, 1, false> plan;
   plan.init(0, lane, a.stk.n, a.dr);
   half_t* const my_k = kt + wave * T::kTileHalves;

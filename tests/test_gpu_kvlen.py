@@ -247,3 +247,58 @@ def test_hf_hook_padding_under_gradient_checkpointing_matches_eager(padding):
         rel = ((grads["fa_p100"][n] - g).norm() / g.norm()).item()
         env_g = ((grads["sdpa"][n] - g).norm() / g.norm()).item()
         assert rel <= max(5e-2, 2 * env_g), (n, rel, env_g)
+
+
+def fill_padding(t, lens):
+    """t (B, H, N, D) with rows lens[b].. of entry b NaN and infinite, as an
+    uninitialised cache may hold them."""
+    t = t.clone()
+    for b, n in enumerate(lens):
+        t[b, :, n::2] = float("nan")
+        t[b, :, n + 1::2] = float("inf")
+    return t
+
+
+PADDED = [
+    # B, Hq, Hkv, N, Nk, D, causal
+    (2, 8, 2, 1, 1000, 128, True),     # decoding, one part
+    (2, 8, 2, 1, 9000, 128, True),     # decoding, parts
+    (3, 8, 2, 5, 900, 256, False),
+    (4, 8, 2, 517, 517, 64, False),    # waves of 32 rows: 4 of them
+    (3, 16, 16, 700, 700, 128, True),
+    (7, 12, 12, 589, 589, 128, True),  # ... long and short tiles paired
+    (9, 16, 8, 134, 134, 64, False),   # 8 waves
+    (12, 16, 4, 138, 138, 256, True),
+    (1, 8, 1, 1188, 5122, 128, True),  # parts
+    (10, 4, 1, 207, 3429, 64, True),   # 8 waves, parts
+    (2, 8, 8, 300, 300, 64, True),     # waves that split the keys
+]
+
+
+@pytest.mark.parametrize("feature", ["plain", "bias", "alibi", "dropout"])
+@pytest.mark.parametrize("B,Hq,Hkv,N,Nk,D,causal", PADDED)
+def test_forward_ignores_nan_and_infinity_past_the_length(B, Hq, Hkv, N, Nk, D, causal, feature):
+    """Only keys [0, kv_len[b]) exist: whatever the rows past them hold, the
+    output is the one of zeros there, bit for bit, in every forward kernel."""
+    import fa_p100
+    if feature in ("bias", "dropout") and (N != Nk or (feature == "bias" and D > 128)):
+        pytest.skip("not with key rows of their own, nor a bias past width 128")
+    g = torch.Generator().manual_seed(N + D)
+    q, k, v = (torch.randn(B, h, n, D, generator=g).half().to(DEV)
+               for h, n in ((Hq, N), (Hkv, Nk), (Hkv, Nk)))
+    lens = [max(1, Nk - 13 - 37 * b) for b in range(B)]
+    kw = dict(kv_len=torch.tensor(lens, dtype=torch.int32, device=DEV))
+    if feature == "bias":  # (N a multiple of 4 takes fa_rows.hip's copy)
+        N = Nk = N // 4 * 4
+        q, k, v = (t[:, :, :N].contiguous() for t in (q, k, v))
+        lens = [min(n, N) for n in lens]
+        kw["bias"] = torch.randn(1, Hq, N, N, generator=g).to(DEV)
+    elif feature == "alibi":
+        kw["alibi_slopes"] = torch.tensor([2.0 ** (-8.0 * (h + 1) / Hq) for h in range(Hq)]).to(DEV)
+    elif feature == "dropout":
+        kw["drop"], _, kw["drop_scale"] = fa_p100.dropout_bits(3, 0.2, B, Hq, N, DEV)
+    zeros = [fill_padding(t, lens).nan_to_num(0.0, 0.0, 0.0) for t in (k, v)]
+    want = fa_p100._ext.forward_dt(q, *zeros, causal, **kw)
+    got = fa_p100._ext.forward_dt(q, fill_padding(k, lens), fill_padding(v, lens), causal, **kw)
+    for x, y in zip(got, want):
+        assert torch.isfinite(y).all() and torch.equal(x, y)
