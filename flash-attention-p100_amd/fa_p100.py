@@ -27,6 +27,7 @@ import os
 import sysconfig
 
 import torch
+from torch.utils._python_dispatch import is_in_torch_dispatch_mode
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _EXT_NAME = "fa_p100_ext"
@@ -51,6 +52,15 @@ _ext = _load_ext()
 # Rows and keys per block of a block-sparse layout (flash_attn's block_mask).
 BLOCK_SIZE = 128
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _watched():
+    """Whether a compiler, a tracer, a dispatch mode or a functorch transform sees
+    this call as torch operators and Functions: the binding's entries are neither,
+    and a graph recorded over them would hold empty tensors."""
+    return (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+            or is_in_torch_dispatch_mode()
+            or torch._C._functorch.peek_interpreter_stack() is not None)
 
 
 def _bnhd_storage(t):
@@ -349,12 +359,11 @@ def flash_attn(q, k, v, causal=False, full_precision=False, kv_len=None, sliding
         else:
             blocks = pack_blocks(block_mask, q.size(0), q.size(1), k.size(1), q.size(2), causal)
     # Calls without these inputs take the same Function in C++ (no interpreter
-    # between the launches); functorch transforms, tracing and tensor subclasses
-    # stay with the Python one, which they know how to handle or refuse.
+    # between the launches); whatever watches the call and tensor subclasses stay
+    # with the Python one, which they know how to record, handle or refuse.
     if mask is None and drop is None and bias is None and blocks is None \
             and type(q) in _PLAIN and type(k) in _PLAIN and type(v) in _PLAIN \
-            and torch._C._functorch.peek_interpreter_stack() is None \
-            and not torch.compiler.is_compiling():
+            and not _watched():
         start, end = segs if segs is not None else (None, None)
         return _ext.flash_attn(q, k, v, causal, full_precision, kv_len, window, alibi_slopes,
                                start, end, scale)
@@ -447,15 +456,15 @@ def segment_bounds(segment_ids):
     A sequence is a maximal run of equal ids along a row: token i belongs to
     the run [seg_start[b, i], seg_end[b, i]). These are the bounds the kernels
     take (fa_options.seg_start / seg_end in the C ABI). One HIP kernel for int32
-    and int64 ids on the GPU, device-side torch scans for any others; nothing is
-    copied to the host.
+    and int64 ids on the GPU, device-side torch scans for any others and where a
+    tracer, compiler or transform watches; nothing is copied to the host.
     """
     s = segment_ids
     B, N = s.shape
-    # (subclasses and functorch's wrapped tensors have no storage of their own)
-    if s.is_cuda and s.dtype in (torch.int32, torch.int64) and 0 < B <= 1 << 21 \
-            and 0 < N < (1 << 31) - (1 << 16) and type(s) is torch.Tensor \
-            and not torch._C._functorch.is_functorch_wrapped_tensor(s):
+    # (a subclass has no storage of its own)
+    if type(s) is torch.Tensor and not _watched() and s.is_cuda \
+            and s.dtype in (torch.int32, torch.int64) and 0 < B <= 1 << 21 \
+            and 0 < N < (1 << 31) - (1 << 16):
         return tuple(_ext.segment_bounds(s))
     idx = torch.arange(N, device=s.device, dtype=torch.int64).expand(B, N)
     change = s[:, 1:] != s[:, :-1]  # a new run starts at i + 1

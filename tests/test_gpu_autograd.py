@@ -109,6 +109,21 @@ def fa_p100_out(q, k, v):
     return o
 
 
+@pytest.mark.parametrize("layout", ["bhnd", "bnhd"])
+def test_a_traced_call_runs_again_on_new_inputs(layout):
+    """torch.jit.trace records the Python Function as a node: the traced module
+    computes new inputs' outputs and their gradients."""
+    import fa_p100
+    first, (q, k, v, do) = leaves(layout, seed=1), leaves(layout, seed=2)
+    traced = torch.jit.trace(lambda q, k, v: fa_p100.flash_attn(q, k, v, True),
+                             tuple(t.detach() for t in first[:3]), check_trace=False)
+    o, want = traced(q, k, v), fa_p100.flash_attn(q, k, v, True)
+    assert torch.equal(o, want)
+    for x, y in zip(torch.autograd.grad(o, (q, k, v), do),
+                    torch.autograd.grad(want, (q, k, v), do)):
+        assert torch.equal(x, y)
+
+
 def test_gradients_on_a_side_stream_and_from_threads():
     import threading
 

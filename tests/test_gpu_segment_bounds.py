@@ -28,3 +28,22 @@ def test_kernel_equals_torch_scans(N, dtype):
             rows_b = b if a.size(0) == b.size(0) else b[:1].expand(3, N)
             assert a.dtype == torch.int32 and a.is_contiguous()
             assert torch.equal(a.cpu(), rows_b)
+
+
+@pytest.mark.parametrize("how", ["jit.trace", "make_fx", "make_fx pre_dispatch", "compile"])
+def test_recorded_and_compiled_calls_stay_torch_operators(how):
+    """A graph recorded over one packing computes another's bounds; a compiled
+    call stays whole."""
+    import fa_p100
+    from torch.fx.experimental.proxy_tensor import make_fx
+    first = (torch.arange(130, device="cuda") // 50).expand(2, 130).contiguous()
+    ids = (torch.arange(130, device="cuda") // 30).expand(2, 130).contiguous()
+    want = fa_p100.segment_bounds(ids)
+    if how == "jit.trace":
+        got = torch.jit.trace(fa_p100.segment_bounds, (first,), check_trace=False)(ids)
+    elif how == "compile":
+        got = torch.compile(fa_p100.segment_bounds, backend="eager", fullgraph=True)(ids)
+    else:
+        got = make_fx(fa_p100.segment_bounds, pre_dispatch=how.endswith("dispatch"))(first)(ids)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
