@@ -622,7 +622,9 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
     return packed_nc ? max(0, min(sst[j], j)) : 0;
   };
   const size_t kv_off = (size_t)(b * stk.b + hkv * stk.h);
-  const rsrc_t rk = rows_rsrc(K + kv_off, NK, stk.n, dr), rv = rows_rsrc(V + kv_off, NK, stk.n, dr);
+  // (rows from the key length on read as zeros: their P is zero, but zero times a
+  // NaN or an infinity that the padding holds would be NaN)
+  const rsrc_t rk = rows_rsrc(K + kv_off, Nk, stk.n, dr), rv = rows_rsrc(V + kv_off, Nk, stk.n, dr);
   // Offset of query head hq's row 0 in Q, dO, dQ.
   auto q_off = [&](int hq) { return (size_t)(b * stq.b + hq * stq.h); };
   constexpr bool MASKB = Feat<FI>::kMask, DROPB = Feat<FI>::kDrop, BIAS = Feat<FI>::kBias;
@@ -739,11 +741,11 @@ __attribute__((amdgpu_waves_per_eu((FEAT & kBwdW4) != 0 ? 2 : 1))) void bwd_kern
         plan_kv.part(vres, rv, tp0, wave, u);
       }
     }
-    if constexpr (KG) {  // this lane's K row j_col (keys past NK: zeros, all masked)
-      const half_t* krow = K + kv_off + (size_t)min(j_col, NK - 1) * stk.n + h * 8;
+    if constexpr (KG) {  // this lane's K row j_col (keys past Nk: zeros, all masked)
+      const half_t* krow = K + kv_off + (size_t)min(j_col, Nk - 1) * stk.n + h * 8;
 #pragma unroll
       for (int kk = 0; kk < D / 16; ++kk)
-        w.kb[kk] = as_half8(load16(krow + kk * 16, j_col < NK && kk * 16 + h * 8 < dr));
+        w.kb[kk] = as_half8(load16(krow + kk * 16, j_col < Nk && kk * 16 + h * 8 < dr));
     }
 #pragma unroll
     for (int k = 0; k < 2 * (D / 32); ++k) w.acc[k] = zero16();

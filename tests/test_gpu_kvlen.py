@@ -302,3 +302,39 @@ def test_forward_ignores_nan_and_infinity_past_the_length(B, Hq, Hkv, N, Nk, D, 
     got = fa_p100._ext.forward_dt(q, fill_padding(k, lens), fill_padding(v, lens), causal, **kw)
     for x, y in zip(got, want):
         assert torch.isfinite(y).all() and torch.equal(x, y)
+
+
+@pytest.mark.parametrize("feature", ["plain", "bias", "alibi", "dropout", "mask"])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal", [
+    (2, 4, 2, 300, 64, True), (2, 4, 4, 390, 128, False), (3, 12, 12, 700, 64, False),
+    (2, 16, 1, 385, 96, True), (2, 4, 2, 300, 256, True), (1, 2, 2, 200, 256, False)])
+def test_backward_ignores_nan_and_infinity_past_the_length(B, Hq, Hkv, N, D, causal, feature):
+    """Gradients with NaN and infinity in the padded keys and values are those
+    of zeros there, bit for bit; padded rows' own are zero."""
+    import fa_p100
+    if feature == "bias" and D > 128:
+        pytest.skip("no bias past width 128")
+    g = torch.Generator().manual_seed(N + D)
+    q, k, v, do = (torch.randn(B, h, N, D, generator=g).half().to(DEV) for h in (Hq, Hkv, Hkv, Hq))
+    lens = [max(1, N - 13 - 137 * b) for b in range(B)]
+    kw = dict(kv_len=torch.tensor(lens, dtype=torch.int32, device=DEV))
+    if feature == "bias":
+        kw["attn_bias"] = torch.randn(1, Hq, N, N, generator=g).to(DEV).requires_grad_()
+    elif feature == "alibi":
+        kw["alibi_slopes"] = torch.tensor([2.0 ** (-8.0 * (h + 1) / Hq) for h in range(Hq)]).to(DEV)
+    elif feature == "dropout":
+        kw.update(dropout_p=0.2, dropout_seed=5)
+    elif feature == "mask":
+        kw["attn_mask"] = (torch.rand(N, N, generator=g) < 0.9).to(DEV)
+    zeros = [fill_padding(t, lens).nan_to_num(0.0, 0.0, 0.0) for t in (k, v)]
+    grads = []
+    for kk, vv in (zeros, [fill_padding(t, lens) for t in (k, v)]):
+        leaves = [t.clone().requires_grad_(True) for t in (q, kk, vv)]
+        if feature == "bias":
+            leaves.append(kw["attn_bias"])
+        o = fa_p100.flash_attn(*leaves[:3], causal, **kw)
+        grads.append(torch.autograd.grad(o, leaves, do))
+    for x, y in zip(*grads):
+        assert torch.isfinite(x).all() and torch.equal(x, y)
+    for b, n in enumerate(lens):
+        assert not any(t[b, :, n:].any() for t in grads[1][1:3])
