@@ -237,9 +237,9 @@ static int fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   const int rc = fwd_args(q, k, v, o, lse, B, Hq, Hkv, N, D, causal, op, stream, a);
   if (rc != FA_OK) return rc;
   if (!q || !k || !v || !o || !lse) return FA_ERR_NULL;
-  if (workspace && workspace_bytes < fa::fwd_workspace_bytes(fa::fwd_plan(a), D))
-    return FA_ERR_WORKSPACE;
-  return to_code(fa::launch_fwd(a, workspace));
+  const fa::FwdPlan plan = fa::fwd_plan(a, workspace != nullptr);
+  if (workspace && workspace_bytes < fa::fwd_workspace_bytes(plan, D)) return FA_ERR_WORKSPACE;
+  return to_code(fa::launch_fwd(a, plan, workspace));
 }
 
 int fa_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B, int Hq,
@@ -266,7 +266,22 @@ size_t fa_fwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int causal,
   if (fwd_args(nullptr, nullptr, nullptr, nullptr, nullptr, B, Hq, Hkv, N, D, causal,
                opts ? *opts : kDefaultOpts, nullptr, a) != FA_OK)
     return 0;
-  return fa::fwd_workspace_bytes(fa::fwd_plan(a), D);
+  return fa::fwd_workspace_bytes(fa::fwd_plan(a, true), D);
+}
+
+int fa_fwd_plan(int B, int Hq, int Hkv, int N, int D, int causal, const fa_options* opts,
+                int workspace, int plan[4]) {
+  fa::FwdArgs a{};
+  const int rc = fwd_args(nullptr, nullptr, nullptr, nullptr, nullptr, B, Hq, Hkv, N, D, causal,
+                          opts ? *opts : kDefaultOpts, nullptr, a);
+  if (rc != FA_OK) return rc;
+  if (!plan) return FA_ERR_NULL;
+  const fa::FwdPlan p = fa::fwd_plan(a, workspace != 0);
+  plan[0] = p.kind;
+  plan[1] = p.waves;
+  plan[2] = p.pair;
+  plan[3] = p.parts;
+  return FA_OK;
 }
 
 int fa_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,

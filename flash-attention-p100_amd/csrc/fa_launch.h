@@ -203,7 +203,8 @@ struct FwdPlan {
   // kv head (kDec), and in all.
   int tiles, items;
 };
-FwdPlan fwd_plan(const FwdArgs& a);
+// workspace: the call has one (else parts is 1).
+FwdPlan fwd_plan(const FwdArgs& a, bool workspace);
 inline size_t part_ml_bytes(const FwdPlan& p) {  // (max, sum) per row of each part
   return align256((size_t)p.items * p.parts * 32 * 8);
 }
@@ -226,8 +227,8 @@ template <int W, bool BF>
 hipError_t launch_bwd_pre_w(const BwdArgs& a);
 template <int W, bool BF>
 hipError_t launch_bwd_main_w(const BwdArgs& a);
-// workspace: fwd_workspace_bytes(fwd_plan(a)) bytes, or null (no parts).
-hipError_t launch_fwd(const FwdArgs& a, void* workspace);
+// workspace: fwd_workspace_bytes(plan) bytes; unused without parts.
+hipError_t launch_fwd(const FwdArgs& a, const FwdPlan& plan, void* workspace);
 hipError_t launch_bwd_preprocess(const BwdArgs& a);
 hipError_t launch_bwd_main(const BwdArgs& a);
 // Dense boolean mask (P planes of N x N bytes) to the bit layouts of

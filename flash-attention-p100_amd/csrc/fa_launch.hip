@@ -208,7 +208,7 @@ double ceil_div(double a, double b) { return ceil(a / b); }
 
 }  // namespace
 
-FwdPlan fwd_plan(const FwdArgs& a) {
+FwdPlan fwd_plan(const FwdArgs& a, bool workspace) {
   FwdPlan best{FwdPlan::kTiles, 0, false, 1, 0, 0};
   // fa_rows.hip takes dropout, a bias (whose rows load 16 bytes at a time) or
   // ALiBi alone, the first two at widths up to 128; the other per-score inputs
@@ -261,6 +261,11 @@ FwdPlan fwd_plan(const FwdArgs& a) {
     return parts == 1 ? 0.0 : 5.0 + 0.0137 * items * parts * W / 128;
   };
   const bool split = NK > a.N && !a.seg_start;  // square calls' results do not depend on a workspace
+  // Without a workspace the search is over one part only: a kernel that is the
+  // best one with several parts can be far from it with one (B=1 H=32/8 N=512,
+  // 8192 keys, D=128 causal: 182 us on 8 waves of fa_rows.hip, 111 on
+  // fa_dec.hip, 138 on fa_fwd.hip).
+  const bool shared = split && workspace;
   constexpr int kTried[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
   {  // fa_rows.hip
     for (const int waves : {4, 8}) {
@@ -271,7 +276,7 @@ FwdPlan fwd_plan(const FwdArgs& a) {
       const FwdTimes& t = waves == 4 ? kRows4Times[wi] : kRows8Times[wi];
       if (n * BH * 512 > kMostItems) continue;
       for (const int parts : kTried) {
-        if (parts > 16 || (parts > 1 && (!split || last < 2 * parts || items * parts > 8192))) break;
+        if (parts > 16 || (parts > 1 && (!shared || last < 2 * parts || items * parts > 8192))) break;
         const double us = a.causal && n > 1 ? uneven_time(t, n * BH * parts, total, last / parts)
                                             : equal_time(t, n * BH * parts, ceil(last / parts), 1);
         consider({FwdPlan::kRows, waves, false, parts, (int)(n * waves), (int)items},
@@ -292,7 +297,7 @@ FwdPlan fwd_plan(const FwdArgs& a) {
     const double seen = keys(a.N, a.N), read = 4.0 * a.B * a.Hkv * seen * a.D / 6.0e6;
     if (items * (W / 32) * 512 <= kMostItems) {
       for (const int parts : kTried) {
-        if (parts > 1 && (seen < 128.0 * parts || items * parts > 8192)) break;
+        if (parts > 1 && (!shared || seen < 128.0 * parts || items * parts > 8192)) break;
         const double rounds = ceil_div(ceil_div(seen, parts), W > 128 ? 128 : 256) * kDecTimes[wi];
         const double n = items * parts, full = floor(n / kCUs), rest = n - full * kCUs;
         double us = full * (rounds * 1.36 + 1.3);
@@ -305,9 +310,7 @@ FwdPlan fwd_plan(const FwdArgs& a) {
   return best;
 }
 
-hipError_t launch_fwd(const FwdArgs& a, void* workspace) {
-  FwdPlan plan = fwd_plan(a);
-  if (!workspace) plan.parts = 1;
+hipError_t launch_fwd(const FwdArgs& a, const FwdPlan& plan, void* workspace) {
   const bool bf = a.dtype == kBF16;
   const hipError_t e = by_width(a, bf, [&](auto w, auto bf, const FwdArgs& a) {
     constexpr int W = decltype(w)::value;

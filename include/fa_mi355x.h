@@ -310,6 +310,10 @@ typedef struct fa_options {
 int fa_fwd_ex(const void* q, const void* k, const void* v, void* o, float* lse,
               int B, int Hq, int Hkv, int N, int D, int causal, const fa_options* opts,
               void* stream);
+int fa_bwd_ex(const void* q, const void* k, const void* v, const void* dO, const void* o,
+              const float* lse, void* dq, void* dk, void* dv, void* workspace,
+              size_t workspace_bytes, int B, int Hq, int Hkv, int N, int D, int causal,
+              const fa_options* opts, void* stream);
 
 /*
  * fa_fwd_ex with a workspace: a call over few query rows (KV-cache decoding,
@@ -326,10 +330,17 @@ size_t fa_fwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D, int causal,
 int fa_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, void* workspace,
               size_t workspace_bytes, int B, int Hq, int Hkv, int N, int D, int causal,
               const fa_options* opts, void* stream);
-int fa_bwd_ex(const void* q, const void* k, const void* v, const void* dO, const void* o,
-              const float* lse, void* dq, void* dk, void* dv, void* workspace,
-              size_t workspace_bytes, int B, int Hq, int Hkv, int N, int D, int causal,
-              const fa_options* opts, void* stream);
+/*
+ * How a forward call would run, from the same arguments (host only: pointers of
+ * `opts` are not read through): plan[0] = 0 for waves that split a tile's keys, 1
+ * for waves of 32 query rows each, 2 for tiles of a kv head's few rows; plan[1] =
+ * waves of a workgroup (kind 1, else 0); plan[2] = 1 where a workgroup takes a
+ * long and a short causal tile; plan[3] = workgroups that share a row's keys (1
+ * when `workspace` is 0: a call without one). Returns what the call would for
+ * invalid arguments. For tests and measurements; no counterpart in the reference.
+ */
+int fa_fwd_plan(int B, int Hq, int Hkv, int N, int D, int causal, const fa_options* opts,
+                int workspace, int plan[4]);
 
 /*
  * Bit-packs a dense boolean mask for fa_options.mask / mask_t. No counterpart

@@ -65,6 +65,12 @@ def load_capi():
     lib.fa_fwd_ex.restype = i
     lib.fa_bwd_ex.argtypes = [vp] * 10 + [sz] + [i] * 6 + [opts, vp]
     lib.fa_bwd_ex.restype = i
+    lib.fa_fwd_workspace_bytes.argtypes = [i] * 6 + [opts]
+    lib.fa_fwd_workspace_bytes.restype = sz
+    lib.fa_fwd_ws.argtypes = [vp] * 6 + [sz] + [i] * 6 + [opts, vp]
+    lib.fa_fwd_ws.restype = i
+    lib.fa_fwd_plan.argtypes = [i] * 6 + [opts, i, ctypes.POINTER(i)]
+    lib.fa_fwd_plan.restype = i
     lib.fa_pack_mask.argtypes = [vp, i, i, vp, vp, vp]
     lib.fa_pack_mask.restype = i
     lib.fa_dropout_bits.argtypes = [ctypes.c_uint64, ctypes.c_float, i, i, vp, vp, vp]

@@ -307,3 +307,38 @@ def test_bnhd_limit_spans_every_head_of_a_row():
     n_max = (2**31 - 1) // (32 * 128) - 256
     assert lib.fa_fwd_bnhd(z, z, z, z, z, 1, 32, 8, n_max, 128, 1, s) == 10005
     assert lib.fa_fwd_bnhd(z, z, z, z, z, 1, 32, 8, n_max + 1, 128, 1, s) == 10007
+
+
+def test_forward_plan_without_a_workspace_is_a_plan_of_one_part():
+    """A call without a workspace takes the best kernel for one part, not the
+    kernel that is the best one with several."""
+    import itertools
+    lib = load_capi()
+
+    def plan(shape, causal, workspace, **kw):
+        out = (ctypes.c_int * 4)()
+        assert lib.fa_fwd_plan(*shape, causal, fa_opts(**kw), workspace, out) == 0
+        return tuple(out)
+
+    shape = (1, 32, 8, 512, 128)
+    assert plan(shape, 1, 1, kv_rows=8192)[3] > 1  # a chunk of a prompt: parts ...
+    kernel, waves, _, parts = plan(shape, 1, 0, kv_rows=8192)
+    assert parts == 1 and (kernel, waves) != (1, 8)  # ... and 64 workgroups of 8 waves are too few
+    differ = 0
+    for B, N, kv, D, causal in itertools.product((1, 4), (1, 33, 512, 1200), (700, 9000),
+                                                 (64, 128, 256), (0, 1)):
+        if kv <= N:
+            continue
+        shape, kw = (B, 8, 2, N, D), dict(kv_rows=kv)
+        none = plan(shape, causal, 0, **kw)
+        assert none[3] == 1
+        nbytes = lib.fa_fwd_workspace_bytes(*shape, causal, fa_opts(**kw))
+        some = plan(shape, causal, 1, **kw)
+        assert (nbytes > 0) == (some[3] > 1)
+        differ += none != some
+    assert differ  # (and square calls take one plan either way)
+    for N, causal in itertools.product((100, 4096), (0, 1)):
+        assert plan((2, 8, 8, N, 64), causal, 0) == plan((2, 8, 8, N, 64), causal, 1)
+    out = (ctypes.c_int * 4)()
+    assert lib.fa_fwd_plan(1, 4, 3, 8, 64, 0, None, 0, out) == 10003
+    assert lib.fa_fwd_plan(1, 4, 2, 8, 64, 0, None, 0, None) == 10005

@@ -80,10 +80,7 @@ def test_capi_workspace():
     refuses a smaller one; without one, fa_fwd_ex's result."""
     import fa_p100
     lib = load_capi()
-    vp, i = ctypes.c_void_p, ctypes.c_int
-    lib.fa_fwd_workspace_bytes.restype = ctypes.c_size_t
-    lib.fa_fwd_workspace_bytes.argtypes = [i] * 6 + [vp]
-    lib.fa_fwd_ws.argtypes = [vp] * 6 + [ctypes.c_size_t] + [i] * 6 + [vp, vp]
+    vp = ctypes.c_void_p
     B, Hq, Hkv, N, Nk, D = 1, 8, 2, 1, 6000, 128
     q, k, v = (t.to(DEV) for t in inputs(B, Hq, Hkv, N, Nk, D, seed=2))
     op = fa_opts(kv_rows=Nk)
@@ -94,8 +91,8 @@ def test_capi_workspace():
     o, lse = torch.empty_like(q), torch.empty(B, Hq, N, device=DEV)
     s = vp(torch.cuda.current_stream().cuda_stream)
     ptrs = [vp(t.data_ptr()) for t in (q, k, v, o, lse)]
-    assert lib.fa_fwd_ws(*ptrs, ws.data_ptr(), size - 1, *args, op, s) == 10006
-    assert lib.fa_fwd_ws(*ptrs, ws.data_ptr(), size, *args, op, s) == 0
+    assert lib.fa_fwd_ws(*ptrs, vp(ws.data_ptr()), size - 1, *args, op, s) == 10006
+    assert lib.fa_fwd_ws(*ptrs, vp(ws.data_ptr()), size, *args, op, s) == 0
     want, want_lse = fa_p100._ext.forward_dt(q, k, v, True)
     assert torch.equal(o, want) and torch.equal(lse, want_lse)
     assert lib.fa_fwd_ws(*ptrs, None, 0, *args, op, s) == 0
