@@ -22,9 +22,9 @@
 //
 // Dropout (FEAT kFeatDrop): a lane's keep bits of the next stage (two words of
 // its row) load during this one. Bias (kFeatBias): each wave's 32 x 64 values of
-// the next stage load into LDS of its own as soon as this stage's are in the
-// score accumulators, which they initialise (fa_fwd.hip reads them per lane
-// from rows N floats apart, 32 cache lines per load).
+// the next stage load into LDS of its own as soon as this stage's are in
+// registers (fa_fwd.hip reads them per lane from rows N floats apart, 32 cache
+// lines per load).
 #include <type_traits>
 
 #include "fa_device.h"
@@ -207,8 +207,11 @@ void rows_kernel(const RowsArgs a) {
         if constexpr (BIAS) bload(min(j + 1, last - 1));
         return;
       }
-      floatx16 s[2];
-      if constexpr (BIAS) {
+      floatx16 s[2] = {zero16(), zero16()}, bv[2];
+      // The bias is added to the finished products (kept in the accumulators from
+      // the start, every product would round at its magnitude). Up to width 64
+      // there are registers to read it before them.
+      auto bread = [&] {
         const float* brow = bt + wave * 32 * kKeys + l32 * kKeys;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -217,15 +220,13 @@ void rows_kernel(const RowsArgs a) {
             const floatx4 x =
                 *reinterpret_cast<const floatx4*>(brow + (((8 * t + 2 * g + h) ^ l32) & 15) * 4);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) s[t][4 * g + e] = x[e] * a.bias_raw;
+            for (int e = 0; e < 4; ++e) bv[t][4 * g + e] = x[e];
           }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // the reads are done before the loads below
         __builtin_amdgcn_sched_barrier(0);
         bload(min(j + 1, last - 1));
-      } else {
-        s[0] = zero16();
-        s[1] = zero16();
-      }
+      };
+      if constexpr (BIAS && D <= 64) bread();
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
 #pragma unroll
@@ -236,6 +237,13 @@ void rows_kernel(const RowsArgs a) {
       }
 #pragma unroll
       for (int u = 2 * (D / 16); u < 2 * kParts; ++u) issue(u);
+      if constexpr (BIAS) {
+        if constexpr (D > 64) bread();
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) s[t][e] = fmaf(bv[t][e], a.bias_raw, s[t][e]);
+      }
       if constexpr (ALIBI) {  // -slope |i - j|, distances exact in fp32
         const float d0 = (float)(i_row + kofs - base - 4 * h);
 #pragma unroll

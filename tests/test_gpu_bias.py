@@ -13,6 +13,7 @@ ABI bit-identical to the op; and Qwen3 through the hook with an additive 4-D mas
 against eager and sdpa. Bars: the fp16 ones (helpers.py) for o, LSE and
 every gradient, dbias included."""
 import ctypes
+import math
 
 import numpy as np
 import pytest
@@ -217,3 +218,43 @@ def test_hf_hook_additive_bias_mask_matches_eager():
     fa = logits("fa_p100")
     env, gap = (sdpa - eager).abs(), (fa - eager).abs()
     assert gap.mean() <= 2 * env.mean() + 1e-4, (gap.mean().item(), env.mean().item())
+
+
+@pytest.mark.parametrize("B,H,N,D", [
+    (8, 12, 516, 64),    # a wave per 32 rows (16-byte bias rows)
+    (2, 32, 388, 128),
+    (4, 8, 301, 64),     # waves that split the keys
+])
+def test_a_large_offset_of_a_row_costs_one_rounding(B, H, N, D):
+    """A bias far larger than the scores is added to them once: the output's
+    error is that of the same call without the offset and one rounding of the
+    score (raw units: bias * sqrt(D)) at the offset's magnitude, which moves
+    the output by as much as the logit. 1.3 times the two for the spread; the
+    products' sum rounded at each of its D / 16 steps gives about 1.9 times.
+    The gradients also see the LSE rounded at that magnitude (in the forward,
+    and as lse * log2(e))."""
+    import fa_p100
+    g = torch.Generator().manual_seed(N)
+    q, k, v, do = (torch.randn(B, H, N, D, generator=g).half().to(DEV) for _ in range(4))
+    small = torch.randn(1, H, N, N, generator=g).to(DEV)
+    rows = torch.empty(1, H, N, 1).uniform_(-11000.0, -8500.0, generator=g).to(DEV)
+
+    def errors(bias):
+        leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        o = fa_p100.flash_attn(*leaves, True, attn_bias=bias)
+        got = (o.detach(), *torch.autograd.grad(o, leaves, do))
+        ref = [t.double().requires_grad_(True) for t in (q, k, v)]
+        s = ref[0] @ ref[1].transpose(-1, -2).contiguous() / D ** 0.5 + bias.double()
+        s = s.masked_fill(torch.ones(N, N, dtype=torch.bool, device=DEV).triu(1), -float("inf"))
+        ro = s.softmax(-1) @ ref[2]
+        want = (ro.detach(), *torch.autograd.grad(ro, ref, do.double()))
+        return [((a.double() - b).norm() / b.norm()).item() for a, b in zip(got, want)]
+
+    base, far = errors(small), errors(small + rows)
+    ulp = lambda x: 2.0 ** (math.floor(math.log2(x)) - 23)
+    score = ulp(11000.0 * D ** 0.5) / math.sqrt(12 * D)
+    lse = math.sqrt(ulp(11000.0) ** 2 + (ulp(11000.0 * math.log2(math.e)) * math.log(2)) ** 2 * 2)
+    lse /= math.sqrt(12)
+    assert far[0] <= 1.3 * math.hypot(base[0], score), (far[0], base[0], score)
+    for x, b in zip(far[1:], base[1:]):
+        assert x <= 1.3 * math.sqrt(b * b + score * score + lse * lse), (x, b, score, lse)
