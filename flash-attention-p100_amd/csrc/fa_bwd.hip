@@ -1212,7 +1212,7 @@ hipError_t launch_main_d(const BwdArgs& a) {
   // equal mask add a key tile's steps in one order, bit for bit, which parts of
   // unequal lists would not.)
   const BwdPlan plan = bwd_plan(a.B, a.Hq, a.Hkv, a.N, key_rows(a.N, a.Nkv), a.D, a.causal,
-                                D == 64 && feat == 0, a.slots != nullptr);
+                                D == 64 && feat == 0, a.shared);
   auto run = [&](auto bounds_tag, auto f) {
     constexpr bool BOUNDS = decltype(bounds_tag)::value;
     constexpr int F = decltype(f)::value;

@@ -96,7 +96,9 @@ const char* fa_error_string(int err) {
     case FA_ERR_HEADS: return "query heads (H) must be a multiple of key/value heads (Hkv)";
     case FA_ERR_BATCH: return "B must be positive";
     case FA_ERR_NULL: return "a required pointer is NULL";
-    case FA_ERR_WORKSPACE: return "workspace is smaller than fa_bwd_workspace_bytes()";
+    case FA_ERR_WORKSPACE:
+      return "workspace is smaller than fa_bwd_workspace_bytes() or, in the forward, "
+             "fa_fwd_workspace_bytes()";
     case FA_ERR_TOO_LARGE: return "shape exceeds the kernels' index range";
     case FA_ERR_LAYOUT: return "layout must be FA_LAYOUT_BHND or FA_LAYOUT_BNHD";
     case FA_ERR_DTYPE: return "unsupported element format";
@@ -332,11 +334,18 @@ int fa_bwd_preprocess(const void* dO, const void* o, const float* lse, void* wor
                  stream);
 }
 
-// Shared by the main-kernel entry points: fp32 dq or 16-bit dq16.
-// workspace_bytes: kChecked where the caller has compared it.
-static constexpr size_t kChecked = SIZE_MAX;
+// What a backward workspace of this size holds the slots of: too little for any
+// call, the causal split's, or those of shared key tiles as well.
+enum Slots { kNoSlots, kPairSlots, kAllSlots };
+static Slots slots_in(size_t bytes, int B, int Hq, int Hkv, int N, int D) {
+  if (bytes < fa::bwd_pair_workspace_bytes(B, Hq, Hkv, N, D)) return kNoSlots;
+  return bytes < fa::bwd_workspace_bytes(B, Hq, Hkv, N, D) ? kPairSlots : kAllSlots;
+}
+
+// Shared by the main-kernel entry points: fp32 dq or 16-bit dq16. `slots`: the
+// workspace's slots_in.
 static int bwd_main(const void* q, const void* k, const void* v, const void* dO,
-                    void* workspace, size_t workspace_bytes, float* dq, void* dq16,
+                    void* workspace, Slots slots, float* dq, void* dq16,
                     void* dk, void* dv, int B, int Hq, int Hkv, int N, int D, int causal,
                     const fa_options& op, void* stream) {
   int rc = check_opts(op, causal, Hq, N, D, true);
@@ -345,8 +354,7 @@ static int bwd_main(const void* q, const void* k, const void* v, const void* dO,
   if (rc == FA_OK) rc = check_kv_rows(op, B, Hq, Hkv, N, D);
   if (rc != FA_OK) return rc;
   if (!q || !k || !v || !dO || !workspace || !(dq || dq16) || !dk || !dv) return FA_ERR_NULL;
-  if (workspace_bytes != kChecked && workspace_bytes < fa::bwd_workspace_bytes(B, Hq, Hkv, N, D))
-    return FA_ERR_WORKSPACE;
+  if (slots == kNoSlots) return FA_ERR_WORKSPACE;
   const fa::BwdWorkspace w = fa::bwd_workspace(B, Hq, N);
   char* ws = static_cast<char*>(workspace);
   fa::BwdArgs a{};
@@ -359,6 +367,7 @@ static int bwd_main(const void* q, const void* k, const void* v, const void* dO,
   a.counters = reinterpret_cast<unsigned*>(ws + w.counters);
   a.n_counters = w.n_counters;
   a.slots = reinterpret_cast<float*>(ws + w.slots);
+  a.shared = slots == kAllSlots;
   a.dq = dq;
   a.dq16 = dq16;
   a.dk = dk;
@@ -404,10 +413,11 @@ static int bwd_16(const void* q, const void* k, const void* v, const void* dO, c
   if (rc == FA_OK) rc = check_kv_rows(op, B, Hq, Hkv, N, D);
   if (rc != FA_OK) return rc;
   if (!workspace || !dq) return FA_ERR_NULL;
-  if (workspace_bytes < fa_bwd_workspace_bytes(B, Hq, Hkv, N, D)) return FA_ERR_WORKSPACE;
+  const Slots slots = slots_in(workspace_bytes, B, Hq, Hkv, N, D);
+  if (slots == kNoSlots) return FA_ERR_WORKSPACE;
   rc = bwd_pre(dO, o, lse, workspace, workspace_bytes, B, Hq, N, D, op.layout, op.dtype, stream);
   if (rc != FA_OK) return rc;
-  return bwd_main(q, k, v, dO, workspace, kChecked, nullptr, dq, dk, dv, B, Hq, Hkv, N, D,
+  return bwd_main(q, k, v, dO, workspace, slots, nullptr, dq, dk, dv, B, Hq, Hkv, N, D,
                   causal, op, stream);
 }
 
@@ -415,7 +425,11 @@ int fa_bwd_main(const void* q, const void* k, const void* v, const void* dO, voi
                 size_t workspace_bytes, float* dq, void* dk, void* dv, int B, int Hq, int Hkv,
                 int N, int D, int causal, void* stream) {
   if (!dq) return FA_ERR_NULL;
-  return bwd_main(q, k, v, dO, workspace, workspace_bytes, dq, nullptr, dk, dv, B, Hq, Hkv, N, D,
+  // (an invalid shape is refused before the slots are looked at)
+  const Slots slots = check_shape(B, Hq, Hkv, N, D) == FA_OK
+                          ? slots_in(workspace_bytes, B, Hq, Hkv, N, D)
+                          : kNoSlots;
+  return bwd_main(q, k, v, dO, workspace, slots, dq, nullptr, dk, dv, B, Hq, Hkv, N, D,
                   causal, kDefaultOpts, stream);
 }
 
@@ -452,11 +466,12 @@ int fa_bwd(const void* q, const void* k, const void* v, const void* dO, const vo
   const int rc = check_shape(B, Hq, Hkv, N, D);
   if (rc != FA_OK) return rc;
   if (!workspace) return FA_ERR_NULL;
-  if (workspace_bytes < fa_bwd_workspace_bytes(B, Hq, Hkv, N, D)) return FA_ERR_WORKSPACE;
+  const Slots slots = slots_in(workspace_bytes, B, Hq, Hkv, N, D);
+  if (slots == kNoSlots) return FA_ERR_WORKSPACE;
   int e = fa_bwd_preprocess(dO, o, lse, workspace, workspace_bytes, B, Hq, N, D, stream);
   if (e != FA_OK) return e;
   if (!dq) return FA_ERR_NULL;
-  return bwd_main(q, k, v, dO, workspace, kChecked, dq, nullptr, dk, dv, B, Hq, Hkv, N, D, causal,
+  return bwd_main(q, k, v, dO, workspace, slots, dq, nullptr, dk, dv, B, Hq, Hkv, N, D, causal,
                   kDefaultOpts, stream);
 }
 
@@ -547,7 +562,8 @@ int fa_bwd_noalloc(const void* q, const void* k, const void* v, const void* dO, 
                                             true).parts *
                        B * Hkv * ((N + fa::kBwdTile - 1) / fa::kBwdTile) *
                        fa::bwd_slot_floats(D) * sizeof(float);
-  a.slots = 2 * vec + slots <= kScratchBytes ? ws + 2 * vec / sizeof(float) : nullptr;
+  a.shared = 2 * vec + slots <= kScratchBytes;
+  a.slots = a.shared ? ws + 2 * vec / sizeof(float) : nullptr;
   a.dq = dq;
   a.B = B;
   a.Hq = Hq;

@@ -105,8 +105,8 @@ struct BwdPlan {
   int parts;   // (apart) workgroups that share one key tile's phase 1
   bool w4;     // width 64: the two-workgroups-per-CU shape
 };
-// has_w4: the launch has such an instantiation; slots: it has the slots of
-// bwd_workspace for NK == N.
+// has_w4: the launch has such an instantiation; slots: it has bwd_workspace_bytes'
+// slots (NK == N), so that parts may be more than one.
 BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, bool has_w4,
                  bool slots);
 // The most parts bwd_plan takes for a shape, whatever the call's options.
@@ -130,12 +130,18 @@ inline BwdWorkspace bwd_workspace(int B, int Hq, int N) {
   w.slots = w.counters + align256((size_t)w.n_counters * sizeof(unsigned));
   return w;
 }
-inline size_t bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D) {
+// With the causal split's slots, two per pair.
+inline size_t bwd_pair_workspace_bytes(int B, int Hq, int Hkv, int N, int D) {
   const int pairs_per_head = ((N + kBwdTile - 1) / kBwdTile) / 2;
-  // Slots: two per pair (the causal split), or one per part of each key tile.
+  return bwd_workspace(B, Hq, N).slots +
+         (size_t)B * Hkv * pairs_per_head * 2 * bwd_slot_floats(D) * sizeof(float);
+}
+// ... or, where that is more, with one per part of each key tile.
+inline size_t bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D) {
+  const size_t pairs = bwd_pair_workspace_bytes(B, Hq, Hkv, N, D);
   const int parts = bwd_max_parts(B, Hq, Hkv, N, D);
-  size_t per_head = (size_t)pairs_per_head * 2;
-  if (parts > 1) per_head = (size_t)parts * ((N + kBwdTile - 1) / kBwdTile);
+  if (parts <= 1) return pairs;
+  const size_t per_head = (size_t)parts * ((N + kBwdTile - 1) / kBwdTile);
   return bwd_workspace(B, Hq, N).slots +
          (size_t)B * Hkv * per_head * bwd_slot_floats(D) * sizeof(float);
 }
@@ -162,6 +168,7 @@ struct BwdArgs {
   // Workspace: partial dK/dV of shared key tiles. Null: every key tile's phase
   // 1 stays in its own workgroup. Null counters turn the causal split off.
   float* slots = nullptr;
+  bool shared = false;  // the slots suffice for the parts of bwd_plan
   int dtype = kFP16;             // of q, k, v, dO, o, dk, dv and dq16
   const int* kv_len = nullptr;   // as FwdArgs::kv_len
   int window = 0;                // as FwdArgs::window

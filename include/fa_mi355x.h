@@ -117,8 +117,11 @@ int fa_fwd_bnhd(const void* q, const void* k, const void* v, void* o, float* lse
  * for each (b, kv head): two for each of those floor(ceil(N/128)/2) pairs of
  * 128-row key tiles (the backward's causal load balancing splits a key tile's
  * work between two workgroups), or, where small grids share every key tile
- * among up to 24 workgroups, one for each of them.
- * Each part is rounded up to 256 bytes. 0 for an invalid shape.
+ * among up to 24 workgroups, one for each of them (the most over causal and
+ * dense calls of the shape: up to about 150 MB). Each part is rounded up to 256
+ * bytes. 0 for an invalid shape. A workspace that ends after the pairs' slots is
+ * taken too: key tiles are then not shared, which is slower on small grids, dq
+ * is the same and dk, dv may differ in the last bits.
  */
 size_t fa_bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D);
 

@@ -3,11 +3,13 @@ key tiles shared by several workgroups, two workgroups per CU and one item per
 tile, each at shapes whose plan takes it, with ragged edges, against the
 float64 oracle at the suite's bars. No counterpart in the reference, which has
 one backward grid (flash_bwd.cuh:475-483)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from helpers import FWD_MAX_ABS, GRAD_REL_L2, REF_REL, make_inputs, np64
+from helpers import FWD_MAX_ABS, GRAD_REL_L2, REF_REL, load_capi, make_inputs, np64
 from oracle import attention as ora
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +82,38 @@ def test_shared_tiles_with_nan_workspace():
     got = fa_p100._ext.backward_dt(q, k, v, do, o, lse, True)
     for a, b in zip(got, ref):
         assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("Hq,Hkv,N,D,causal", [
+    (16, 1, 500, 64, True), (16, 1, 900, 128, False), (4, 2, 300, 256, True)])
+def test_a_workspace_of_the_pairs_slots_is_enough(Hq, Hkv, N, D, causal):
+    """A workspace that ends after two slots per pair of key tiles is taken: the
+    same dQ bit for bit, dK and dV up to the order of their sums, no byte past
+    it touched; one byte less is refused."""
+    lib = load_capi()
+    q, k, v, do = (t.to(DEV) for t in make_inputs(1, Hq, Hkv, N, D, seed=7))
+    o, lse = torch.empty_like(q), torch.empty(1, Hq, N, device=DEV)
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    shape = (1, Hq, Hkv, N, D, int(causal))
+    assert lib.fa_fwd(*map(p, (q, k, v, o, lse)), *shape, 0, s) == 0
+    a256 = lambda n: (n + 255) // 256 * 256
+    pairs = -(-N // 128) // 2
+    width = next(w for w in (32, 64, 96, 128, 256) if D <= w)
+    small = 2 * a256(Hq * N * 4) + a256(Hq * pairs * 4) + Hkv * pairs * 2 * 128 * width * 2 * 4
+    full = lib.fa_bwd_workspace_bytes(*shape[:5])
+    assert small < full
+    grads = []
+    for size in (full, small):
+        ws = torch.full((full // 4 + 64,), float("nan"), device=DEV)
+        out = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        args = [*map(p, (q, k, v, do, o, lse, *out)), p(ws)]
+        assert lib.fa_bwd_half_dq(*args, size, *shape, s) == 0
+        assert torch.isnan(ws[size // 4:]).all()
+        grads.append(out)
+    assert lib.fa_bwd_half_dq(*args, small - 1, *shape, s) == 10006
+    assert torch.equal(grads[0][0], grads[1][0])
+    for x, y in zip(*grads):
+        assert torch.isfinite(x).all()
+        # (fp32 sums in another order, rounded to 16 bits: an ulp here and there)
+        assert ((x.float() - y.float()).norm() / x.float().norm()).item() <= 2 ** -11
