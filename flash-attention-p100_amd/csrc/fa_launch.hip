@@ -227,7 +227,7 @@ FwdPlan fwd_plan(const FwdArgs& a, bool workspace) {
     const double hi = a.causal ? fmax(1, fmin(NK, i1 + kofs)) : NK;
     return a.window > 0 ? fmin(hi, rows + a.window) : hi;
   };
-  double least;
+  double least, one_tile;  // (one_tile: workgroups of one 64-row tile)
   {  // fa_fwd.hip
     const double n = ceil_div(a.N, 64), stage = W > 128 ? 64 : 128;
     const bool pairs = a.causal && n > 1;
@@ -236,17 +236,28 @@ FwdPlan fwd_plan(const FwdArgs& a, bool workspace) {
     const double steps = 0.5 * (first + last) * n * BH / wgs, tiles = pairs ? 2 : 1;
     const FwdTimes& t = kTilesTimes[wi];
     const bool masked = a.N % 64 || a.kv_len || a.window > 0 || a.alibi || a.seg_start || NK != a.N;
+    one_tile = a.causal ? HUGE_VAL : wgs;
     least = 1 + (kTilesW4[wi] > 0 && wgs >= 2 * kCUs && !(a.causal && masked)
                      ? wgs / (2 * kCUs) * (steps * kTilesW4[wi] + tiles * t.ends)
                      : equal_time(t, wgs, steps, tiles));
   }
   // These inputs cost the two kernels differently: a bias takes fa_fwd.hip 2.6
   // times as long as none and fa_rows.hip 1.6 times (B=4 H=8 N=1024 D=64 dense:
-  // 51 -> 28 us, B=1 H=16 N=4096 D=64 causal: 217 -> 136, B=2 H=32 N=1500 D=128
-  // causal: 185 -> 125); dropout costs fa_rows.hip more than fa_fwd.hip's unmasked
+  // 51 -> 28 us, B=1 H=16 N=4096 D=64 causal: 217 -> 127, B=2 H=32 N=1500 D=128
+  // causal: 185 -> 120); dropout costs fa_rows.hip more than fa_fwd.hip's unmasked
   // copies (79 us there and 82 here at B=1 H=16 N=4096 D=64 causal) and as much as
   // its masked ones, which a ragged N takes (96 -> 72 us at B=2 H=32 N=1500 D=128).
-  if (a.bias) least *= 1.6;
+  // Dense grids of at most one tile per CU gain nothing from waves of 32 rows at
+  // the widths from 128 on, whose estimate there is 15-20% high, nor with a bias
+  // (up to width 64: on half as many tiles): 28.7 us against 37.0 at B=1 H=2 N=1396
+  // D=96, 14.7 against 17.9 at B=2 H=4 N=400 D=128 with one, 17.0 against 20.4 at
+  // B=4 H=4 N=260 D=256 without. Of 1400 random calls with a bias 99 ran more than
+  // 5% slower than on fa_fwd.hip without this rule, 4 with it.
+  const double few = a.bias && W <= 64 ? kCUs / 2 : kCUs;
+  if (one_tile <= few && NK == a.N && !a.seg_start)
+    least *= a.bias ? (W <= 64 ? 1.0 : W <= 96 ? 0.9 : 0.8) : (W <= 96 ? 1.0 : W <= 128 ? 0.85 : 0.8);
+  else if (a.bias)
+    least *= 1.6;
   if (a.drop && a.N % 128 == 0) least *= 0.85;
   // A launch's work-items and the row blocks' indices stay within 32 bits.
   constexpr double kMostItems = 4294967295.0;

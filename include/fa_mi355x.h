@@ -48,7 +48,7 @@ enum {
   FA_ERR_HEADS = 10003,      /* Hkv <= 0 or Hq % Hkv != 0 (fa_p100_ext.cu:61, 113) */
   FA_ERR_BATCH = 10004,      /* B <= 0 */
   FA_ERR_NULL = 10005,       /* a required pointer is NULL */
-  FA_ERR_WORKSPACE = 10006,  /* workspace smaller than fa_bwd_workspace_bytes() */
+  FA_ERR_WORKSPACE = 10006,  /* workspace too small (fa_bwd_ / fa_fwd_workspace_bytes()) */
   FA_ERR_TOO_LARGE = 10007,  /* (N+256)*D (BNHD: (N+256)*H*D) over 2^31-1, or over 2^29 for a
                                 head dim that is not 32, 64, 96, 128 or 256; or a launch's work
                                 items over 2^32 */
