@@ -1208,11 +1208,7 @@ hipError_t launch_main_d(const BwdArgs& a) {
                       a.seg_start != nullptr || key_rows(a.N, a.Nkv) != a.N;
   const int feat = feat_of(a.mask != nullptr, a.drop != nullptr, a.bias != nullptr,
                            a.block_rows != nullptr);
-  // (A mask and a block layout run with one item per tile: a layout and the
-  // equal mask add a key tile's steps in one order, bit for bit, which parts of
-  // unequal lists would not.)
-  const BwdPlan plan = bwd_plan(a.B, a.Hq, a.Hkv, a.N, key_rows(a.N, a.Nkv), a.D, a.causal,
-                                D == 64 && feat == 0, a.shared);
+  const BwdPlan plan = bwd_plan(a);
   auto run = [&](auto bounds_tag, auto f) {
     constexpr bool BOUNDS = decltype(bounds_tag)::value;
     constexpr int F = decltype(f)::value;

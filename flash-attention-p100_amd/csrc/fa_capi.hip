@@ -298,6 +298,46 @@ size_t fa_bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D) {
   return fa::bwd_workspace_bytes(B, Hq, Hkv, N, D);
 }
 
+// What a backward workspace of this size holds the slots of: too little for any
+// call, the causal split's, or those of shared key tiles as well.
+enum Slots { kNoSlots, kPairSlots, kAllSlots };
+static Slots slots_in(size_t bytes, int B, int Hq, int Hkv, int N, int D) {
+  if (bytes < fa::bwd_pair_workspace_bytes(B, Hq, Hkv, N, D)) return kNoSlots;
+  return bytes < fa::bwd_workspace_bytes(B, Hq, Hkv, N, D) ? kPairSlots : kAllSlots;
+}
+
+int fa_bwd_plan(int B, int Hq, int Hkv, int N, int D, int causal, const fa_options* opts,
+                size_t workspace_bytes, int plan[3]) {
+  const fa_options& op = opts ? *opts : kDefaultOpts;
+  int rc = check_opts(op, causal, Hq, N, D, true);
+  if (rc == FA_OK) rc = check_shape(B, Hq, Hkv, N, D);
+  if (rc == FA_OK && op.layout == fa::kBNHD) rc = check_bnhd(Hq, N, D);
+  if (rc == FA_OK) rc = check_kv_rows(op, B, Hq, Hkv, N, D);
+  if (rc != FA_OK) return rc;
+  if (!plan) return FA_ERR_NULL;
+  const Slots slots = slots_in(workspace_bytes, B, Hq, Hkv, N, D);
+  if (slots == kNoSlots) return FA_ERR_WORKSPACE;
+  fa::BwdArgs a{};
+  a.B = B;
+  a.Hq = Hq;
+  a.Hkv = Hkv;
+  a.N = N;
+  a.D = D;
+  a.causal = causal != 0;
+  a.window = op.window;
+  a.mask = op.mask;
+  a.drop = op.drop;
+  a.bias = op.bias;
+  a.Nkv = op.kv_rows;
+  a.block_rows = op.block_rows;
+  a.shared = slots == kAllSlots;
+  const fa::BwdPlan p = fa::bwd_plan(a);
+  plan[0] = p.apart;
+  plan[1] = p.parts;
+  plan[2] = p.w4;
+  return FA_OK;
+}
+
 static int bwd_pre(const void* dO, const void* o, const float* lse, void* workspace,
                    size_t workspace_bytes, int B, int Hq, int N, int D, int layout, int dtype,
                    void* stream) {
@@ -332,14 +372,6 @@ int fa_bwd_preprocess(const void* dO, const void* o, const float* lse, void* wor
                       size_t workspace_bytes, int B, int Hq, int N, int D, void* stream) {
   return bwd_pre(dO, o, lse, workspace, workspace_bytes, B, Hq, N, D, fa::kBHND, fa::kFP16,
                  stream);
-}
-
-// What a backward workspace of this size holds the slots of: too little for any
-// call, the causal split's, or those of shared key tiles as well.
-enum Slots { kNoSlots, kPairSlots, kAllSlots };
-static Slots slots_in(size_t bytes, int B, int Hq, int Hkv, int N, int D) {
-  if (bytes < fa::bwd_pair_workspace_bytes(B, Hq, Hkv, N, D)) return kNoSlots;
-  return bytes < fa::bwd_workspace_bytes(B, Hq, Hkv, N, D) ? kPairSlots : kAllSlots;
 }
 
 // Shared by the main-kernel entry points: fp32 dq or 16-bit dq16. `slots`: the
@@ -558,8 +590,8 @@ int fa_bwd_noalloc(const void* q, const void* k, const void* v, const void* dO, 
   a.lse2 = ws + vec / sizeof(float);
   a.counters = nullptr;
   a.n_counters = 0;
-  const size_t slots = (size_t)fa::bwd_plan(B, Hq, Hkv, N, N, D, causal != 0, D > 32 && D <= 64,
-                                            true).parts *
+  const size_t slots = (size_t)fa::bwd_plan(B, Hq, Hkv, N, N, D, causal != 0, 0,
+                                            D > 32 && D <= 64, true).parts *
                        B * Hkv * ((N + fa::kBwdTile - 1) / fa::kBwdTile) *
                        fa::bwd_slot_floats(D) * sizeof(float);
   a.shared = 2 * vec + slots <= kScratchBytes;

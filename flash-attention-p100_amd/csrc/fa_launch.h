@@ -107,8 +107,8 @@ struct BwdPlan {
 };
 // has_w4: the launch has such an instantiation; slots: it has bwd_workspace_bytes'
 // slots (NK == N), so that parts may be more than one.
-BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, bool has_w4,
-                 bool slots);
+BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, int window,
+                 bool has_w4, bool slots);
 // The most parts bwd_plan takes for a shape, whatever the call's options.
 int bwd_max_parts(int B, int Hq, int Hkv, int N, int D);
 struct BwdWorkspace {
@@ -235,6 +235,14 @@ hipError_t launch_bwd_pre_w(const BwdArgs& a);
 template <int W, bool BF>
 hipError_t launch_bwd_main_w(const BwdArgs& a);
 // workspace: fwd_workspace_bytes(plan) bytes; unused without parts.
+// The plan of a main-kernel launch. (A mask and a block layout run with one item
+// per tile: a layout and the equal mask add a key tile's steps in one order, bit
+// for bit, which parts of unequal lists would not.)
+inline BwdPlan bwd_plan(const BwdArgs& a) {
+  if (a.mask || a.block_rows) return {false, 1, false};
+  const bool w4 = padded_head_dim(a.D) == 64 && !a.drop && !a.bias;
+  return bwd_plan(a.B, a.Hq, a.Hkv, a.N, key_rows(a.N, a.Nkv), a.D, a.causal, a.window, w4, a.shared);
+}
 hipError_t launch_fwd(const FwdArgs& a, const FwdPlan& plan, void* workspace);
 hipError_t launch_bwd_preprocess(const BwdArgs& a);
 hipError_t launch_bwd_main(const BwdArgs& a);

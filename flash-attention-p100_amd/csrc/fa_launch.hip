@@ -1,6 +1,7 @@
 // The tile width of a launch, and the sizes of the launches it makes.
 #include "fa_launch.h"
 
+#include <limits.h>
 #include <math.h>
 
 #include <type_traits>
@@ -40,13 +41,21 @@ hipError_t by_width(const Args& a, bool bf, const Launch& launch) {
 // the longest phase-1 item then bounds a grid of one round (B=1 H=8 N=4096
 // D=128: 136 us against 132 together). Parts cut that item, which with few kv
 // heads or rows is most of the time, for the price of writing and summing the
-// partials. The constants were fitted to 7638 timed plans of 1183 random shapes
-// (64 <= D <= 256, 100 <= N <= 8192, B <= 16, 1 to 64 heads): the plan taken is
-// 1.4% slower than the best one on average, one item per tile 46% slower.
-// Backward, same box, together -> apart: 1042 -> 948 us (the ragged dense shape
-// above); 180 -> 131 at B=2 H=8 N=2663 D=128 causal; with parts 737 -> 113 (8
-// parts) at B=1 H=16/1 N=2048 D=128 causal, 512 -> 396 (4) at B=1 H=32/4 N=4608
-// D=64 causal, 321 -> 146 (4) at B=3 H=16/4 N=896 D=256 causal.
+// partials. The constants were fitted to 7638 timed plans of 1183 random square
+// shapes (64 <= D <= 256, 100 <= N <= 8192, B <= 16, 1 to 64 heads) without a
+// window: the plan taken is 1.4% slower than the best one on average, one item per
+// tile 46% slower. Over 1400 random calls each, the plan taken is 1.3% slower than
+// the best with a window and 0.6% with unequal sides (3.9% and 2.3% before they
+// were priced); 2% of the calls are more than 5% slower than one item per tile.
+// Key lengths and packed sequences are on the device, so the plan does not see
+// them (1.7% and 3.6%); a mask's, dropout's and a bias's cost is not in it either
+// (a bias: 2.9%). Backward, same box, one item per tile -> the plan's: 1102 -> 974
+// us (the ragged dense shape above, apart); 162 -> 126 at B=2 H=8 N=2663 D=128
+// causal (apart); 720 -> 110 at B=1 H=16/1 N=2048 D=128 causal (16 parts), 529 ->
+// 403 at B=1 H=32/4 N=4608 D=64 causal (4), 312 -> 154 at B=3 H=16/4 N=896 D=256
+// causal (3); 32 -> 22 at B=3 H=1 N=3801 D=128, window 107 (39 with the 3 parts
+// that the whole triangle would get); 184 -> 144 at B=5 H=4/2 N=3581, 807 keys,
+// D=64 (290 on two workgroups per CU).
 namespace {
 
 constexpr int kPartsTried[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
@@ -54,9 +63,11 @@ constexpr int kPartsTried[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
 struct BwdCost {
   int W, G;
   double nk, nq, n1, n2, total;  // tiles of a head, items of the phases, all units
-  bool causal;
+  double q_reach, k_reach;       // most query tiles a key tile is seen by, key tiles one sees
+  bool causal, window;
 
-  BwdCost(int B, int Hq, int Hkv, int N, int NK, int D, bool causal) : causal(causal) {
+  BwdCost(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, int window)
+      : causal(causal), window(window > 0) {
     W = padded_head_dim(D);
     G = Hq / Hkv;
     nk = (NK + kBwdTile - 1) / kBwdTile;
@@ -64,7 +75,17 @@ struct BwdCost {
     n1 = (double)B * Hkv * nk;
     n2 = (double)B * Hq * nq;
     const double half = 0.5 * nq * (nq + 1);  // causal, the last rows aligned
-    const double blocks = !causal ? nk * nq : nk >= nq ? nq * (nk - nq) + half : 0.5 * nk * (nk + 1);
+    double blocks = !causal ? nk * nq : nk >= nq ? nq * (nk - nq) + half : 0.5 * nk * (nk + 1);
+    q_reach = causal ? fmin(nq, nk) : nq;
+    k_reach = nk;
+    if (window > 0) {  // (in streamed tiles of 64 rows, half a tile each)
+      const double reach = (ceil((window - 1) / 64.0) + 2) / 2;
+      q_reach = fmin(q_reach, reach);
+      k_reach = fmin(k_reach, reach);
+      // Query tiles see lo .. nk key tiles, at most `reach` of them.
+      const double lo = fmax(1.0, nk - nq + 1), below = fmax(lo - 1, floor(fmin(reach, nk)));
+      blocks = 0.5 * (lo + below) * (below - lo + 1) + (nk - below) * reach;
+    }
     total = 7.0 * B * Hq * blocks;
   }
   // Units of a block's product and of an item's start and end, at this width;
@@ -78,13 +99,20 @@ struct BwdCost {
   static constexpr double kSolo = 0.8;  // a workgroup alone on its CU, of unit(true)
 
   double together(bool w4) const {
-    const double n = nk > nq ? n1 : n1 * nq / nk;
-    // (width 256 and unequal sides run without the causal split)
-    const double item =
-        unit(w4) * (causal && (W > 128 || nk != nq) ? G * (4.0 * nq + 3.0) : total / n);
+    const double n = nk > nq ? n1 : n1 * nq / nk, slots = w4 ? 2 * kCUs : kCUs;
     const double ends = fixed(w4) * (1.0 + 0.46 * G);
+    if (nk != nq) {  // workgroups with both phases beside workgroups with one
+      const double item = G * (4.0 * q_reach + 3.0 * k_reach) * unit(w4);
+      return fmax(total * unit(w4) / fmin(slots, n), item * (w4 && n <= kCUs ? kSolo : 1.0)) +
+             ends * ceil(n / slots) + (n > slots ? 0.5 * item : 0.0);
+    }
+    // (width 256 and windows run without the causal split)
+    const double item =
+        unit(w4) * (window ? G * (4.0 * q_reach + 3.0 * fmin(fmax(nk - q_reach + 1, 1.0), k_reach))
+                    : causal && W > 128 ? G * (4.0 * nq + 3.0)
+                                        : total / n);
     if (!w4) return ceil(n / kCUs) * (item + ends);
-    const double full = floor(n / (2 * kCUs)), rest = n - full * 2 * kCUs;
+    const double full = floor(n / slots), rest = n - full * slots;
     const double last = rest <= 0 ? 0.0 : item * (rest > kCUs ? 1.0 : kSolo) + ends;
     return full * (item + ends) + last;
   }
@@ -92,9 +120,10 @@ struct BwdCost {
     const double items = n1 * parts + n2, u = unit(w4), slots = w4 ? 2 * kCUs : kCUs;
     const double ends = 0.77 * fixed(w4), work = total * u + items * ends;
     const bool few = w4 && items < slots;
-    double t = fmax(work / slots, 4.0 * G * nq * u / parts * (few ? kSolo : 1.0) + ends);
+    double t = fmax(work / slots, 4.0 * G * q_reach * u / parts * (few ? kSolo : 1.0) + ends);
     if (few) t = fmax(t, work / kCUs * kSolo);
-    if (items > slots) t += 0.36 * 3.0 * (causal ? 0.5 * nk : nk) * u;  // the uneven end
+    if (items > slots)  // the uneven end
+      t += 0.36 * 3.0 * (window ? k_reach : causal ? 0.5 * nk : nk) * u;
     if (parts > 1) t += 1.0 + 0.17 * n1 * parts * (W / 128.0);
     return 1.03 * t;  // (one item per tile where the two are about equal)
   }
@@ -105,9 +134,12 @@ struct BwdCost {
 
 }  // namespace
 
-BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, bool has_w4,
-                 bool slots) {
-  const BwdCost cost(B, Hq, Hkv, N, NK, D, causal);
+BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, int window,
+                 bool has_w4, bool slots) {
+  const BwdCost cost(B, Hq, Hkv, N, NK, D, causal, window);
+  // One item per tile, two workgroups per CU where the grid fills both.
+  const BwdPlan plain{false, 1,
+                      has_w4 && fmax(cost.nk, cost.nq) * (double)B * Hkv >= 2.0 * kCUs};
   BwdPlan best{false, 1, false};
   double least = HUGE_VAL;
   auto consider = [&](BwdPlan p, double t) {
@@ -116,12 +148,16 @@ BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, bool
       best = p;
     }
   };
+  // (windows' shared tiles stay within the workspace, which is sized without one)
+  const int most = window > 0 ? bwd_max_parts(B, Hq, Hkv, N, D) : INT_MAX;
   // (a launch counts its work-items in 32 bits: one item per tile always fits)
   const double threads = cost.W > 128 ? 256.0 : 512.0;
   auto search = [&](bool w4, bool may_share) {
+    // Windows and unequal sides: another plan only for a clear gain.
+    if ((window > 0 || cost.nk != cost.nq) && w4 == plain.w4) consider(plain, 0.95 * cost.together(w4));
     consider({false, 1, w4}, cost.together(w4));
     for (const int parts : kPartsTried) {
-      if (parts > 1 && (!may_share || NK != N)) break;
+      if (parts > 1 && (!may_share || NK != N || parts > most)) break;
       if (!cost.allows(parts, N) || (cost.n1 * parts + cost.n2 + 16) * threads > 4294967295.0) break;
       consider({true, parts, w4}, cost.apart(parts, w4));
     }
@@ -140,7 +176,7 @@ int bwd_max_parts(int B, int Hq, int Hkv, int N, int D) {
   for (const bool causal : {false, true})
     for (const bool w4 : {false, true}) {
       if (w4 && padded_head_dim(D) != 64) continue;
-      const BwdPlan p = bwd_plan(B, Hq, Hkv, N, N, D, causal, w4, true);
+      const BwdPlan p = bwd_plan(B, Hq, Hkv, N, N, D, causal, 0, w4, true);
       if (p.parts > most) most = p.parts;
     }
   return most;

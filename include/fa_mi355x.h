@@ -344,6 +344,14 @@ int fa_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, 
  */
 int fa_fwd_plan(int B, int Hq, int Hkv, int N, int D, int causal, const fa_options* opts,
                 int workspace, int plan[4]);
+/*
+ * The same for a backward call with a workspace of that size: plan[0] = 1 where
+ * the passes over key tiles (dK, dV) and over query tiles (dQ) are work items
+ * apart, plan[1] = workgroups that share a key tile, plan[2] = 1 for two
+ * workgroups per CU (width 64).
+ */
+int fa_bwd_plan(int B, int Hq, int Hkv, int N, int D, int causal, const fa_options* opts,
+                size_t workspace_bytes, int plan[3]);
 
 /*
  * Bit-packs a dense boolean mask for fa_options.mask / mask_t. No counterpart

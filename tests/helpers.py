@@ -71,6 +71,8 @@ def load_capi():
     lib.fa_fwd_ws.restype = i
     lib.fa_fwd_plan.argtypes = [i] * 6 + [opts, i, ctypes.POINTER(i)]
     lib.fa_fwd_plan.restype = i
+    lib.fa_bwd_plan.argtypes = [i] * 6 + [opts, sz, ctypes.POINTER(i)]
+    lib.fa_bwd_plan.restype = i
     lib.fa_pack_mask.argtypes = [vp, i, i, vp, vp, vp]
     lib.fa_pack_mask.restype = i
     lib.fa_dropout_bits.argtypes = [ctypes.c_uint64, ctypes.c_float, i, i, vp, vp, vp]

@@ -342,3 +342,40 @@ def test_forward_plan_without_a_workspace_is_a_plan_of_one_part():
     out = (ctypes.c_int * 4)()
     assert lib.fa_fwd_plan(1, 4, 3, 8, 64, 0, None, 0, out) == 10003
     assert lib.fa_fwd_plan(1, 4, 2, 8, 64, 0, None, 0, None) == 10005
+
+
+def test_backward_plan_stays_within_the_workspace():
+    """The slots of every plan, windowed calls' too, fit fa_bwd_workspace_bytes;
+    a workspace of the pairs' slots leaves key tiles unshared, with the same
+    workgroups; masks and block layouts run one item per tile."""
+    import random
+    lib, r, shared = load_capi(), random.Random(5), 0
+    width = lambda D: next(w for w in (32, 64, 96, 128, 256) if D <= w)
+    a256 = lambda n: (n + 255) // 256 * 256
+
+    def plan(shape, causal, nbytes, **kw):
+        out = (ctypes.c_int * 3)()
+        assert lib.fa_bwd_plan(*shape, causal, fa_opts(**kw), nbytes, out) == 0
+        return tuple(out)
+
+    for _ in range(400):
+        B, Hkv, G, N, D = (r.choice(x) for x in ((1, 2, 5, 16), (1, 2, 8), (1, 4, 16),
+                                                 (130, 500, 1024, 3001, 8192), (40, 64, 80, 128, 256)))
+        shape = (B, Hkv * G, Hkv, N, D)
+        nbytes = lib.fa_bwd_workspace_bytes(*shape)
+        tiles, pairs = -(-N // 128), -(-N // 128) // 2
+        slots = 2 * a256(B * Hkv * G * N * 4) + a256(B * Hkv * G * pairs * 4)
+        slot = 128 * width(D) * 2 * 4
+        small = slots + B * Hkv * pairs * 2 * slot
+        for causal, window in ((0, 0), (1, 0), (1, 50), (1, 700)):
+            apart, parts, w4 = plan(shape, causal, nbytes, window=window)
+            assert parts == 1 or slots + B * Hkv * tiles * parts * slot <= nbytes
+            assert apart or parts == 1
+            assert not w4 or width(D) == 64
+            shared += parts > 1
+            assert plan(shape, causal, small, window=window)[1:] == (1, w4)
+        assert plan(shape, 1, nbytes, mask=1, mask_t=1, mask_heads=1) == (0, 1, 0)
+        assert plan(shape, 1, nbytes, block_rows=1, block_cols=1) == (0, 1, 0)
+    assert shared > 100
+    out = (ctypes.c_int * 3)()
+    assert lib.fa_bwd_plan(1, 4, 2, 300, 64, 1, None, 0, out) == 10006
