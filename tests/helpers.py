@@ -119,5 +119,23 @@ def fa_opts(dtype=0, layout=0, kv_len=None, window=0, alibi_slopes=None, seg_sta
     return ctypes.pointer(o)
 
 
+def fwd_plan(B, Hq, Hkv, N, Nk, D, causal, **opts):
+    """(kernel, waves, paired, parts) of a forward call with a workspace: "tiles"
+    (fa_fwd.hip), "rows" (fa_rows.hip) or "dec" (fa_dec.hip); options as fa_opts."""
+    out = (ctypes.c_int * 4)()
+    op = fa_opts(kv_rows=0 if Nk == N else Nk, **opts)
+    assert load_capi().fa_fwd_plan(B, Hq, Hkv, N, D, int(causal), op, 1, out) == 0
+    return ("tiles", "rows", "dec")[out[0]], out[1], bool(out[2]), out[3]
+
+
+def bwd_plan(B, Hq, Hkv, N, D, causal, **opts):
+    """(apart, parts, two workgroups per CU) of a backward call with a workspace of
+    fa_bwd_workspace_bytes; options as fa_opts."""
+    lib, out = load_capi(), (ctypes.c_int * 3)()
+    size = lib.fa_bwd_workspace_bytes(B, Hq, Hkv, N, D)
+    assert lib.fa_bwd_plan(B, Hq, Hkv, N, D, int(causal), fa_opts(**opts), size, out) == 0
+    return bool(out[0]), out[1], bool(out[2])
+
+
 def np64(t):
     return t.detach().cpu().double().numpy()

@@ -1,39 +1,48 @@
 """The backward's work division (bwd_plan, csrc/fa_launch.hip): phases apart,
 key tiles shared by several workgroups, two workgroups per CU and one item per
-tile, each at shapes whose plan takes it, with ragged edges, against the
-float64 oracle at the suite's bars. No counterpart in the reference, which has
-one backward grid (flash_bwd.cuh:475-483)."""
+tile, each at shapes whose plan takes it (asserted: fa_bwd_plan), with ragged
+edges, against the float64 oracle at the suite's bars. No counterpart in the
+reference, which has one backward grid (flash_bwd.cuh:475-483)."""
 import ctypes
 
 import numpy as np
 import pytest
 import torch
 
-from helpers import FWD_MAX_ABS, GRAD_REL_L2, REF_REL, load_capi, make_inputs, np64
+from helpers import (FWD_MAX_ABS, GRAD_REL_L2, REF_REL, bwd_plan, load_capi, make_inputs,
+                     np64)
 from oracle import attention as ora
 
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda"
 
+# B, Hq, Hkv, N, D, causal: apart, parts, two workgroups per CU (bwd_plan)
 CASES = [
-    # B, Hq, Hkv, N, D, causal
-    (1, 4, 4, 256, 64, True),     # apart, one part
-    (1, 16, 1, 385, 64, True),    # parts: one kv head, a ragged last tile
-    (1, 16, 1, 511, 128, False),  # parts, dense ragged (keys past N masked once)
-    (1, 6, 2, 129, 128, True),    # a tile of one row; more parts than steps in it
-    (2, 4, 2, 300, 256, True),    # parts at width 256
-    (1, 8, 2, 300, 96, True),     # parts at width 96
-    (1, 8, 2, 200, 40, False),    # a head dim below its width
-    (3, 12, 12, 700, 64, False),  # two workgroups per CU, apart
-    (9, 8, 8, 537, 128, True),    # over one round of one item per tile, apart
-    (1, 1, 1, 2, 128, True),      # two rows (with one, dQ and dK are zero up to rounding)
+    ((1, 4, 4, 256, 64, True), (True, 1, False)),
+    ((1, 16, 1, 385, 64, True), (True, 16, False)),   # one kv head, a ragged last tile
+    ((1, 16, 1, 511, 128, False), (True, 16, False)),  # keys past N masked once
+    ((1, 6, 2, 129, 128, True), (True, 3, False)),    # a tile of one row; more parts than steps
+    ((2, 4, 2, 300, 256, True), (True, 4, False)),
+    ((1, 8, 2, 300, 96, True), (True, 8, False)),
+    ((1, 8, 2, 200, 40, False), (True, 6, False)),    # a head dim below its width
+    ((3, 12, 12, 700, 64, False), (True, 1, True)),
+    ((5, 8, 2, 774, 64, True), (True, 3, True)),
+    ((11, 4, 1, 387, 64, False), (True, 3, True)),
+    ((9, 8, 8, 537, 128, True), (True, 1, False)),    # over one round of one item per tile
+    ((10, 12, 12, 394, 64, True), (False, 1, True)),
+    ((9, 4, 4, 778, 64, True), (False, 1, False)),    # tiles split in pairs, an odd number
+    ((10, 12, 12, 167, 128, False), (False, 1, False)),
+    ((9, 12, 12, 161, 256, False), (False, 1, False)),
+    ((1, 1, 1, 2, 128, True), (True, 1, False)),  # two rows (with one, dQ and dK are zero up to rounding)
 ]
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal", CASES)
-def test_plans_match_oracle(B, Hq, Hkv, N, D, causal):
+@pytest.mark.parametrize("shape,plan", CASES)
+def test_plans_match_oracle(shape, plan):
     import fa_p100
+    assert bwd_plan(*shape) == plan
+    B, Hq, Hkv, N, D, causal = shape
     q, k, v, do = make_inputs(B, Hq, Hkv, N, D, seed=N + D)
     qg, kg, vg = (t.to(DEV).requires_grad_(True) for t in (q, k, v))
     o = fa_p100.flash_attn(qg, kg, vg, causal)
@@ -70,18 +79,28 @@ def test_key_tiles_past_every_key_length_have_zero_gradients():
             assert g[0, :, :130].any() and g[1, :, 512:].any()
 
 
-def test_shared_tiles_with_nan_workspace():
-    """Slots and outputs hold NaN before the call: every value read was written."""
-    import fa_p100
-    q, k, v, do = (t.to(DEV) for t in make_inputs(1, 16, 1, 500, 64, seed=4))
-    o, lse = fa_p100._ext.forward_dt(q, k, v, True)
-    ref = fa_p100._ext.backward_dt(q, k, v, do, o, lse, True)
-    junk = torch.full((64 << 20,), float("nan"), device=DEV)
-    torch.cuda.synchronize()
-    del junk  # its block serves the next call's workspace
-    got = fa_p100._ext.backward_dt(q, k, v, do, o, lse, True)
-    for a, b in zip(got, ref):
-        assert torch.isfinite(a).all() and torch.equal(a, b)
+@pytest.mark.parametrize("shape,plan", CASES)
+def test_nothing_unwritten_is_read(shape, plan):
+    """Workspace and outputs full of NaN before the call: the results of zeros
+    there, bit for bit, so that every value read was written and every element
+    of the outputs is."""
+    lib = load_capi()
+    B, Hq, Hkv, N, D, causal = shape
+    q, k, v, do = (t.to(DEV) for t in make_inputs(B, Hq, Hkv, N, D, seed=4))
+    o, lse = torch.empty_like(q), torch.empty(B, Hq, N, device=DEV)
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    args = (B, Hq, Hkv, N, D, int(causal))
+    assert lib.fa_fwd(*map(p, (q, k, v, o, lse)), *args, 0, s) == 0
+    size = lib.fa_bwd_workspace_bytes(*args[:5])
+    results = []
+    for fill in (0.0, float("nan")):
+        ws = torch.full((size // 4,), fill, device=DEV)
+        out = [torch.full_like(t, fill) for t in (q, k, v)]
+        assert lib.fa_bwd_half_dq(*map(p, (q, k, v, do, o, lse, *out, ws)), size, *args, s) == 0
+        results.append(out)
+    for a, b in zip(*results):
+        assert torch.isfinite(b).all() and torch.equal(a, b)
 
 
 @pytest.mark.parametrize("Hq,Hkv,N,D,causal", [

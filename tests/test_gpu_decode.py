@@ -9,24 +9,24 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import FWD_MAX_ABS, LSE_MAX_ABS, fa_opts, load_capi, np64
+from helpers import FWD_MAX_ABS, LSE_MAX_ABS, fa_opts, fwd_plan, load_capi, np64
 from oracle import attention as ora
 
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda"
 
+# B, Hq, Hkv, N, Nk, D, causal: parts (fwd_plan)
 CASES = [
-    # B, Hq, Hkv, N, Nk, D, causal
-    (1, 16, 8, 1, 1021, 128, True),    # one part
-    (1, 8, 2, 1, 4097, 128, True),     # parts; a block of one key
-    (2, 8, 1, 4, 3000, 64, True),      # 32 rows of eight heads
-    (1, 8, 1, 5, 2049, 64, False),     # 40 rows: a head across two tiles
-    (1, 4, 4, 33, 1500, 96, True),     # 33 rows of one head
-    (2, 4, 2, 3, 2500, 256, True),     # four waves
-    (1, 2, 1, 2, 1100, 40, True),      # a head dim below its width
-    (3, 1, 1, 1, 2, 128, True),        # two keys: most waves have no block
-    (1, 2, 2, 1, 700, 32, False),
+    ((1, 16, 8, 1, 1021, 128, True), 1),
+    ((1, 8, 2, 1, 4097, 128, True), 24),    # a block of one key
+    ((2, 8, 1, 4, 3000, 64, True), 12),     # 32 rows of eight heads
+    ((1, 8, 1, 5, 2049, 64, False), 12),    # 40 rows: a head across two tiles
+    ((1, 4, 4, 33, 1500, 96, True), 6),     # 33 rows of one head
+    ((2, 4, 2, 3, 2500, 256, True), 12),    # four waves
+    ((1, 2, 1, 2, 1100, 40, True), 1),      # a head dim below its width
+    ((3, 1, 1, 1, 2, 128, True), 1),        # two keys: most waves have no block
+    ((1, 2, 2, 1, 700, 32, False), 1),
 ]
 
 
@@ -45,9 +45,11 @@ def check(o, lse, ref, bf16=False):
 
 
 @pytest.mark.parametrize("dtype", [torch.half, torch.bfloat16])
-@pytest.mark.parametrize("B,Hq,Hkv,N,Nk,D,causal", CASES)
-def test_decode_matches_oracle(B, Hq, Hkv, N, Nk, D, causal, dtype):
+@pytest.mark.parametrize("shape,parts", CASES)
+def test_decode_matches_oracle(shape, parts, dtype):
     import fa_p100
+    assert fwd_plan(*shape) == ("dec", 0, False, parts)
+    B, Hq, Hkv, N, Nk, D, causal = shape
     q, k, v = inputs(B, Hq, Hkv, N, Nk, D, seed=N + Nk, dtype=dtype)
     ref = ora.attention_fwd(*(t.double().numpy() for t in (q, k, v)), causal)
     dense = [t.to(DEV) for t in (q, k, v)]
@@ -58,12 +60,15 @@ def test_decode_matches_oracle(B, Hq, Hkv, N, Nk, D, causal, dtype):
     assert torch.equal(ob.transpose(1, 2), o) and torch.equal(lse_b, lse)
 
 
-@pytest.mark.parametrize("N,Nk,window", [(1, 2000, 0), (1, 2000, 300), (6, 1537, 70)])
-def test_decode_with_key_lengths_window_and_alibi(N, Nk, window):
+@pytest.mark.parametrize("N,Nk,window,parts", [
+    (1, 2000, 0, 8), (1, 2000, 300, 1), (6, 1537, 70, 1), (1, 9000, 5000, 12), (6, 9001, 4000, 16)])
+def test_decode_with_key_lengths_window_and_alibi(N, Nk, window, parts):
     """Lengths from one key to all; with a window some rows see no key (o = 0,
     lse = +inf); parts past an entry's keys are empty."""
     import fa_p100
     B, Hq, Hkv, D = 4, 8, 2, 64
+    assert fwd_plan(B, Hq, Hkv, N, Nk, D, True, kv_len=1, window=window,
+                    alibi_slopes=1) == ("dec", 0, False, parts)
     q, k, v = inputs(B, Hq, Hkv, N, Nk, D, seed=Nk)
     lens = [1, 260, Nk - 3, Nk]
     slopes = torch.tensor([2.0 ** (-h - 1) for h in range(Hq)])

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import FWD_MAX_ABS, GRAD_REL_L2, LSE_MAX_ABS, REF_REL, make_inputs, np64
+from helpers import FWD_MAX_ABS, GRAD_REL_L2, LSE_MAX_ABS, REF_REL, fwd_plan, make_inputs, np64
 from oracle import attention as ora
 
 pytestmark = pytest.mark.gpu
@@ -259,28 +259,30 @@ def fill_padding(t, lens):
     return t
 
 
+# B, Hq, Hkv, N, Nk, D, causal: the kernel, its waves, paired, parts (fwd_plan)
 PADDED = [
-    # B, Hq, Hkv, N, Nk, D, causal
-    (2, 8, 2, 1, 1000, 128, True),     # decoding, one part
-    (2, 8, 2, 1, 9000, 128, True),     # decoding, parts
-    (3, 8, 2, 5, 900, 256, False),
-    (4, 8, 2, 517, 517, 64, False),    # waves of 32 rows: 4 of them
-    (3, 16, 16, 700, 700, 128, True),
-    (7, 12, 12, 589, 589, 128, True),  # ... long and short tiles paired
-    (9, 16, 8, 134, 134, 64, False),   # 8 waves
-    (12, 16, 4, 138, 138, 256, True),
-    (1, 8, 1, 1188, 5122, 128, True),  # parts
-    (10, 4, 1, 207, 3429, 64, True),   # 8 waves, parts
-    (2, 8, 8, 300, 300, 64, True),     # waves that split the keys
+    ((2, 8, 2, 1, 1000, 128, True), ("dec", 0, False, 1)),
+    ((2, 8, 2, 1, 9000, 128, True), ("dec", 0, False, 24)),
+    ((3, 8, 2, 5, 900, 256, False), ("dec", 0, False, 4)),
+    ((4, 8, 2, 517, 517, 64, False), ("rows", 4, False, 1)),
+    ((3, 16, 16, 700, 700, 128, True), ("rows", 4, False, 1)),
+    ((7, 12, 12, 589, 589, 128, True), ("rows", 4, True, 1)),
+    ((3, 48, 12, 130, 130, 64, False), ("rows", 8, False, 1)),
+    ((12, 16, 4, 138, 138, 256, True), ("rows", 8, False, 1)),
+    ((1, 8, 1, 1188, 5122, 128, True), ("rows", 4, False, 3)),
+    ((10, 4, 1, 207, 3429, 64, True), ("rows", 8, False, 6)),
+    ((1, 2, 2, 300, 300, 64, False), ("tiles", 0, False, 1)),
 ]
 
 
 @pytest.mark.parametrize("feature", ["plain", "bias", "alibi", "dropout"])
-@pytest.mark.parametrize("B,Hq,Hkv,N,Nk,D,causal", PADDED)
-def test_forward_ignores_nan_and_infinity_past_the_length(B, Hq, Hkv, N, Nk, D, causal, feature):
+@pytest.mark.parametrize("shape,plan", PADDED)
+def test_forward_ignores_nan_and_infinity_past_the_length(shape, plan, feature):
     """Only keys [0, kv_len[b]) exist: whatever the rows past them hold, the
     output is the one of zeros there, bit for bit, in every forward kernel."""
     import fa_p100
+    B, Hq, Hkv, N, Nk, D, causal = shape
+    assert fwd_plan(*shape, kv_len=1) == plan
     if feature in ("bias", "dropout") and (N != Nk or (feature == "bias" and D > 128)):
         pytest.skip("not with key rows of their own, nor a bias past width 128")
     g = torch.Generator().manual_seed(N + D)

@@ -1,32 +1,44 @@
 """The forward whose waves own 32 rows each (csrc/fa_rows.hip): 4 and 8 waves,
 long and short causal tiles paired, key ranges shared by workgroups, each at
-shapes whose plan takes it (fwd_plan, csrc/fa_launch.hip), with ragged tiles,
+shapes whose plan takes it (asserted: fa_fwd_plan), with ragged tiles,
 key lengths, windows and packed sequences; one (batch, head) slice against the
 float64 oracle (flash_fwd.cuh:321-339 is the result it restates)."""
 import numpy as np
 import pytest
 import torch
 
-from helpers import FWD_MAX_ABS, LSE_MAX_ABS, np64
+from helpers import FWD_MAX_ABS, LSE_MAX_ABS, fwd_plan, np64
 from oracle import attention as ora
 
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda"
 
+# B, Hq, Hkv, N, Nk, D, causal: waves, paired, parts (fwd_plan)
 CASES = [
-    # B, Hq, Hkv, N, Nk, D, causal
-    (2, 4, 2, 264, 264, 80, True),      # 4 waves, a last tile of 8 rows
-    (8, 4, 1, 257, 257, 256, True),     # ... of one row
-    (10, 8, 2, 145, 145, 128, False),   # keys past N masked
-    (14, 12, 12, 189, 189, 64, True),
-    (12, 8, 2, 321, 321, 32, True),
-    (7, 12, 12, 589, 589, 128, False),  # 8 waves
-    (6, 8, 8, 1114, 1114, 256, True),   # 8 waves
-    (4, 8, 8, 3634, 3634, 64, True),    # paired tiles, an odd number of them
-    (8, 4, 4, 3032, 3032, 128, True),   # paired tiles
-    (1, 8, 1, 1188, 5122, 128, True),   # parts
-    (1, 4, 1, 1474, 3529, 256, True),   # parts
+    ((2, 4, 2, 264, 264, 80, True), (4, False, 1)),  # a last tile of 8 rows
+    ((8, 4, 1, 257, 257, 256, True), (4, False, 1)),  # ... of one row
+    ((10, 8, 2, 145, 145, 128, False), (4, False, 1)),  # keys past N masked
+    ((7, 12, 12, 589, 589, 128, False), (4, False, 1)),
+    ((1, 2, 2, 138, 138, 256, False), (4, False, 1)),
+    ((14, 12, 12, 189, 189, 64, True), (8, False, 1)),
+    ((12, 8, 2, 321, 321, 32, True), (8, False, 1)),
+    ((11, 12, 12, 398, 398, 80, True), (8, False, 1)),
+    ((16, 16, 8, 169, 169, 128, True), (8, False, 1)),
+    ((11, 16, 8, 132, 132, 256, True), (8, False, 1)),
+    ((12, 12, 12, 133, 133, 32, False), (8, False, 1)),
+    ((3, 48, 12, 130, 130, 64, False), (8, False, 1)),
+    ((13, 12, 12, 129, 129, 256, False), (8, False, 1)),
+    ((10, 12, 12, 340, 340, 32, True), (4, True, 1)),
+    ((4, 8, 8, 3634, 3634, 64, True), (4, True, 1)),  # an odd number of tiles
+    ((13, 4, 2, 514, 514, 96, True), (4, True, 1)),
+    ((9, 48, 12, 136, 136, 128, True), (4, True, 1)),
+    ((6, 8, 8, 1114, 1114, 256, True), (4, True, 1)),
+    ((1, 8, 1, 1188, 5122, 128, True), (4, False, 3)),
+    ((3, 1, 1, 968, 4668, 96, False), (4, False, 8)),
+    ((6, 4, 4, 680, 3570, 64, False), (8, False, 3)),
+    ((3, 16, 8, 188, 4334, 80, True), (8, False, 4)),
+    ((1, 8, 2, 1474, 6000, 256, True), (8, False, 4)),
 ]
 
 
@@ -48,9 +60,11 @@ def check(o, lse, q, k, v, causal, b, h, bf16=False, **kw):
 
 
 @pytest.mark.parametrize("dtype", [torch.half, torch.bfloat16])
-@pytest.mark.parametrize("B,Hq,Hkv,N,Nk,D,causal", CASES)
-def test_rows_match_oracle(B, Hq, Hkv, N, Nk, D, causal, dtype):
+@pytest.mark.parametrize("shape,plan", CASES)
+def test_rows_match_oracle(shape, plan, dtype):
     import fa_p100
+    assert fwd_plan(*shape) == ("rows", *plan)
+    B, Hq, Hkv, N, Nk, D, causal = shape
     q, k, v = make(B, Hq, Hkv, N, Nk, D, seed=N + D, dtype=dtype)
     dense = [t.to(DEV) for t in (q, k, v)]
     o, lse = fa_p100._ext.forward_dt(*dense, causal)
@@ -63,15 +77,16 @@ def test_rows_match_oracle(B, Hq, Hkv, N, Nk, D, causal, dtype):
 
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("option", ["kv_len", "window", "segments"])
-def test_rows_bounds(option, causal):
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,waves", [
+    (4, 8, 2, 517, 64, 4), (3, 48, 12, 136, 64, 8), (12, 16, 4, 140, 256, 8)])
+def test_rows_bounds(B, Hq, Hkv, N, D, waves, option, causal):
     """Lengths of one key and up; windows narrower than a stage; sequences of
     one token, at a stage's edge and over several tiles."""
     import fa_p100
-    B, Hq, Hkv, N, D = 3, 8, 2, 517, 64
     q, k, v = make(B, Hq, Hkv, N, N, D, seed=8)
     kw, okw = {}, {}
     if option == "kv_len":
-        lens = [1, 64, 300]
+        lens = [min(N, n) for n in ([1, 64, 300, 129] * B)[:B]]
         kw["kv_len"] = torch.tensor(lens, dtype=torch.int32, device=DEV)
         okw = [dict(kv_len=[n]) for n in lens]
     elif option == "window":
@@ -80,19 +95,20 @@ def test_rows_bounds(option, causal):
         kw["window"] = 37
         okw = [dict(window=37)] * B
     else:
-        cuts = [[1, 64, 192, 200, 517], [517], [130, 131, 400, 517]]
-        ids = torch.tensor([[sum(i >= c for c in cs) for i in range(N)] for cs in cuts])
+        cuts = [[1, 64, 192, 200], [], [130, 131, 400]]
+        ids = torch.tensor([[sum(i >= c for c in cuts[b % 3]) for i in range(N)] for b in range(B)])
         kw["seg_start"], kw["seg_end"] = fa_p100.segment_bounds(ids.to(DEV))
         okw = [dict(segments=ids[b:b + 1].numpy()) for b in range(B)]
+    assert fwd_plan(B, Hq, Hkv, N, N, D, causal, **kw) == ("rows", waves, False, 1)
     o, lse = fa_p100._ext.forward_dt(*(t.to(DEV) for t in (q, k, v)), causal, **kw)
-    for b in range(B):
+    for b in range(min(B, 4)):
         check(o, lse, q, k, v, causal, b, Hq - 1, **okw[b])
 
 
 FEAT_CASES = [
     # B, H, N, D, causal: N a multiple of 4 (the bias rows' 16-byte loads), ragged
     # against stages of 64 keys and tiles of 128 rows
-    (4, 8, 300, 64, False),
+    (8, 12, 516, 64, False),
     (8, 12, 516, 64, True),
     (3, 16, 260, 96, True),
     (2, 32, 388, 128, True),
@@ -108,6 +124,8 @@ def test_rows_bias_and_dropout(B, H, N, D, causal, feature):
     head's loads), -inf and the type's lowest value in it, dropout's keep bits,
     and a bias with key lengths."""
     import fa_p100
+    given = dict(drop=1, drop_scale=1.25) if feature == "dropout" else dict(bias=16)
+    assert fwd_plan(B, H, H, N, N, D, causal, **given) == ("rows", 4, N == 1284, 1)
     q, k, v = make(B, H, H, N, N, D, seed=N)
     dev = [t.to(DEV) for t in (q, k, v)]
     g = torch.Generator().manual_seed(1)
@@ -144,36 +162,40 @@ def check_drop(o, lse, q, k, v, causal, b, h, dropout):
     assert ora.max_abs(np64(lse[b:b + 1, h:h + 1]), ref_lse) <= LSE_MAX_ABS
 
 
-def test_bias_gradient_is_written_whole():
+@pytest.mark.parametrize("layout", ["bhnd", "bnhd"])
+@pytest.mark.parametrize("N", [130, 256])
+def test_bias_gradient_is_written_whole(N, layout):
     """Without causal masking, lengths or sequences the backward writes every
-    element of the bias's gradient, into memory that held NaN."""
+    element of the bias's gradient: a buffer of NaN comes back finite."""
     import fa_p100
-    for N in (130, 256):
-        q, k, v, do = (torch.randn(2, 4, N, 64, device=DEV).half() for _ in range(4))
-        bias = torch.randn(1, 4, N, N, device=DEV, requires_grad=True)
-        junk = torch.full((2, 4, N, N), float("nan"), device=DEV)
-        torch.cuda.synchronize()
-        del junk  # its block serves the gradient
-        o = fa_p100.flash_attn(q, k, v, attn_bias=bias)
-        (db,) = torch.autograd.grad(o, bias, do)
-        assert torch.isfinite(db).all()
-        s = (q.float() @ k.float().transpose(-1, -2).contiguous() / 8 + bias.detach())
-        p = s.softmax(-1)
-        dp = do.float() @ v.float().transpose(-1, -2).contiguous()
-        ds = p * (dp - (dp * p).sum(-1, keepdim=True))
-        ref = ds.sum(0, keepdim=True)
-        assert ((db - ref).norm() / ref.norm()).item() <= 5e-3
+    q, k, v, do = (torch.randn(2, 4, N, 64, device=DEV).half() for _ in range(4))
+    bias = torch.randn(1, 4, N, N, device=DEV)
+    dbias = torch.full((2, 4, N, N), float("nan"), device=DEV)
+    forward, backward = fa_p100._ext.forward_dt, fa_p100._ext.backward_dt
+    args = [q, k, v, do]
+    if layout == "bnhd":
+        forward, backward = fa_p100._ext.forward_bnhd, fa_p100._ext.backward_bnhd
+        args = [t.transpose(1, 2).contiguous() for t in args]
+    o, lse = forward(*args[:3], False, bias=bias)
+    backward(*args, o, lse, False, bias=bias, dbias=dbias)
+    assert torch.isfinite(dbias).all()
+    s = (q.float() @ k.float().transpose(-1, -2).contiguous() / 8 + bias)
+    p = s.softmax(-1)
+    dp = do.float() @ v.float().transpose(-1, -2).contiguous()
+    ref = p * (dp - (dp * p).sum(-1, keepdim=True))
+    assert ((dbias - ref).norm() / ref.norm()).item() <= 5e-3
 
 
-@pytest.mark.parametrize("B,H,N,Nk,D,causal", [
-    (4, 8, 300, 300, 64, False),
-    (8, 12, 517, 517, 128, True),
-    (4, 16, 1285, 1285, 64, True),   # paired tiles
-    (3, 16, 261, 261, 256, True),
-    (1, 8, 1188, 5122, 96, True),    # distances from the last key's diagonal
+@pytest.mark.parametrize("B,H,N,Nk,D,causal,plan", [
+    (8, 12, 516, 516, 64, False, (4, False, 1)),
+    (8, 12, 517, 517, 128, True, (4, False, 1)),
+    (4, 16, 1285, 1285, 64, True, (4, True, 1)),
+    (3, 16, 261, 261, 256, True, (4, False, 1)),
+    (1, 8, 1188, 5122, 96, True, (4, False, 3)),  # distances from the last key's diagonal
 ])
-def test_rows_alibi(B, H, N, Nk, D, causal):
+def test_rows_alibi(B, H, N, Nk, D, causal, plan):
     import fa_p100
+    assert fwd_plan(B, H, H, N, Nk, D, causal, alibi_slopes=1) == ("rows", *plan)
     q, k, v = make(B, H, H, N, Nk, D, seed=N)
     slopes = torch.tensor([2.0 ** (-8.0 * (h + 1) / H) for h in range(H)])
     o, lse = fa_p100._ext.forward_dt(*(t.to(DEV) for t in (q, k, v)), causal,

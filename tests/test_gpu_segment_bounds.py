@@ -1,6 +1,6 @@
 """segment_bounds' HIP kernel (fa_segment_bounds) against its torch scans, which
-CPU ids take: rows around a thread's 16 ids and a workgroup's 4096, both id
-types, ids that are not dense. No counterpart in the reference."""
+CPU ids take: rows around a thread's 4 ids, a wave's 256 and a workgroup's
+4096, both id types, ids that are not dense. No counterpart in the reference."""
 import pytest
 import torch
 
@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
-@pytest.mark.parametrize("N", [1, 2, 15, 16, 17, 1024, 4095, 4096, 4097, 9000])
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 255, 256, 257, 1024, 4095, 4096, 4097, 9000])
 def test_kernel_equals_torch_scans(N, dtype):
     import fa_p100
     g = torch.Generator().manual_seed(N)
