@@ -118,7 +118,7 @@ int fa_fwd_bnhd(const void* q, const void* k, const void* v, void* o, float* lse
  * 128-row key tiles (the backward's causal load balancing splits a key tile's
  * work between two workgroups), or, where small grids share every key tile
  * among up to 24 workgroups, one for each of them (the most over causal and
- * dense calls of the shape: up to about 150 MB). Each part is rounded up to 256
+ * dense calls of the shape: up to about 110 MB in all). Each part is rounded up to 256
  * bytes. 0 for an invalid shape. A workspace that ends after the pairs' slots is
  * taken too: key tiles are then not shared, which is slower on small grids, dq
  * is the same and dk, dv may differ in the last bits.
