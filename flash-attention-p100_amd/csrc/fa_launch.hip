@@ -188,14 +188,15 @@ int bwd_max_parts(int B, int Hq, int Hkv, int N, int D) {
 // 1400 random calls each the plan taken is 2.4% slower than the best candidate on
 // average (key lengths, ALiBi and dropout 2%, a bias 0.9%, packed sequences, which
 // it does not see, 5.5%), fa_fwd.hip alone 31% (24% with dropout, 89% with a
-// window). Same box, fa_fwd.hip -> the plan's: 358 -> 312 us at B=2 H=32/8 N=3001 D=128 dense (fa_rows.hip, 4
-// waves), 312 -> 293 at B=1 H=16 N=8192 D=128 causal (4 waves, paired), 248 -> 164
-// at B=9 H=12 N=2145 D=128 causal (4 waves, paired), 21 -> 8.0 at B=14 H=12 N=189
-// D=64 causal (8 waves); fa_fwd.hip stays where few rows leave CUs idle (B=1 H=8
-// N=4096 D=128 causal: 48 us, 73 with 4 waves). More keys than rows: 222 -> 100 at
-// B=16 H=32/8 N=1, 8192 keys, D=128 (fa_dec.hip, 2 parts); 240 -> 30 at B=1 H=32/8
-// N=1, 32768 keys (24 parts); 225 -> 19 at B=1 H=16/2 N=4, 8000 keys, D=256 (32
-// parts); 134 -> 86 at B=1 H=32/8 N=512, 8192 keys (fa_rows.hip, 8 waves, 3 parts).
+// window). Same box, fa_fwd.hip -> the plan's: 358 -> 312 us at B=2 H=32/8 N=3001
+// D=128 dense (fa_rows.hip, 4 waves), 312 -> 293 at B=1 H=16 N=8192 D=128 causal
+// (4 waves, paired), 248 -> 164 at B=9 H=12 N=2145 D=128 causal (the same), 21 ->
+// 8.0 at B=14 H=12 N=189 D=64 causal (8 waves); fa_fwd.hip stays where few rows
+// leave CUs idle (B=1 H=8 N=4096 D=128 causal: 48 us, 73 with 4 waves). More keys
+// than rows: 222 -> 100 at B=16 H=32/8 N=1, 8192 keys, D=128 (fa_dec.hip, 2 parts);
+// 240 -> 30 at B=1 H=32/8 N=1, 32768 keys (24 parts); 225 -> 19 at B=1 H=16/2 N=4,
+// 8000 keys, D=256 (32 parts); 134 -> 86 at B=1 H=32/8 N=512, 8192 keys
+// (fa_rows.hip, 8 waves, 3 parts).
 namespace {
 
 // One kernel's times at a width.
