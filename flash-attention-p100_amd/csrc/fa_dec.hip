@@ -27,7 +27,6 @@ namespace {
 
 constexpr int kRows = 32;             // query rows of a tile
 constexpr int kKeys = 32;             // keys of a wave's block
-constexpr float kRescaleLog2 = 8.f;   // as the forward's lazy rescale
 
 template <int D>
 struct Dec {
@@ -38,12 +37,6 @@ struct Dec {
   static constexpr int kFloats = kRows * D;  // a partial O (one row tile)
   static_assert(kWaves / 2 * kFloats * 4 <= kWaves * kTileHalves * 2, "merge area exceeds the tiles");
 };
-
-__device__ __forceinline__ float max_halves(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
 
 // A wave's LDS reads so far are done: its tile may be loaded again.
 __device__ __forceinline__ void wait_lds() {

@@ -84,6 +84,17 @@ __device__ __forceinline__ half8 as_half8(u32x4 v) {
 // Swap with the lane 32 positions away (the other half of the wave).
 __device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32, 64); }
 
+// Row max over the two half-waves: lanes l and l ^ 32 hold the same query row.
+__device__ __forceinline__ float max_halves(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// Threshold of the forward kernels' lazy rescale: the running sum and O are
+// rescaled only when a row's maximum grows by more than this, in log2 units.
+constexpr float kRescaleLog2 = 8.f;
+
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4v lds_short4;
 

@@ -51,7 +51,6 @@ namespace fa {
 namespace {
 
 constexpr int kBR = 64;    // query rows per tile (2 row blocks of 32)
-constexpr float kRescaleLog2 = 8.f;  // lazy-rescale threshold, log2 units
 
 // Waves and staged keys per width. Up to D = 128: 8 waves (two per SIMD) =
 // 2 row blocks x 4 key quarters of a 128-key stage. At D = 256 a wave's Q
@@ -96,13 +95,6 @@ struct FwdLds {
   static constexpr int kIssueSlots = D / 16 + D / 32;
   static_assert(2 * kEvenParts <= kIssueSlots, "more loads than issue points");
 };
-
-// Row max over the two half-waves: lanes l and l ^ 32 hold the same query row.
-__device__ __forceinline__ float max_halves(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
 
 // QLDS: Q's operands are read from a staged LDS tile (qt, rows qrow ..) at
 // each product instead of being held in registers (qb); the bias copy does

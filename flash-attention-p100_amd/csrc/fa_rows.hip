@@ -34,7 +34,6 @@ namespace fa {
 namespace {
 
 constexpr int kFeatAlibi = 64;  // (a FEAT bit beside Feat's)
-constexpr float kRescaleLog2 = 8.f;  // as the forward's lazy rescale
 
 template <int D, int NW>
 struct Rows {
@@ -43,12 +42,6 @@ struct Rows {
   static constexpr int kKeys = 64;       // keys of a stage
   static constexpr int kTileHalves = TileLoad<D, kKeys, NW>::kHalves;
 };
-
-__device__ __forceinline__ float max_halves(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
 
 struct RowsArgs {
   const half_t* q;
