@@ -330,7 +330,7 @@ int fa_bwd_plan(int B, int Hq, int Hkv, int N, int D, int causal, const fa_optio
   a.bias = op.bias;
   a.Nkv = op.kv_rows;
   a.block_rows = op.block_rows;
-  a.shared = slots == kAllSlots;
+  a.share = slots == kAllSlots ? fa::BwdShare::kShare : fa::BwdShare::kNone;
   const fa::BwdPlan p = fa::bwd_plan(a);
   plan[0] = p.apart;
   plan[1] = p.parts;
@@ -399,7 +399,7 @@ static int bwd_main(const void* q, const void* k, const void* v, const void* dO,
   a.counters = reinterpret_cast<unsigned*>(ws + w.counters);
   a.n_counters = w.n_counters;
   a.slots = reinterpret_cast<float*>(ws + w.slots);
-  a.shared = slots == kAllSlots;
+  a.share = slots == kAllSlots ? fa::BwdShare::kShare : fa::BwdShare::kNone;
   a.dq = dq;
   a.dq16 = dq16;
   a.dk = dk;
@@ -591,11 +591,12 @@ int fa_bwd_noalloc(const void* q, const void* k, const void* v, const void* dO, 
   a.counters = nullptr;
   a.n_counters = 0;
   const size_t slots = (size_t)fa::bwd_plan(B, Hq, Hkv, N, N, D, causal != 0, 0,
-                                            D > 32 && D <= 64, true).parts *
+                                            D > 32 && D <= 64, fa::BwdShare::kShare).parts *
                        B * Hkv * ((N + fa::kBwdTile - 1) / fa::kBwdTile) *
                        fa::bwd_slot_floats(D) * sizeof(float);
-  a.shared = 2 * vec + slots <= kScratchBytes;
-  a.slots = a.shared ? ws + 2 * vec / sizeof(float) : nullptr;
+  const bool shared = 2 * vec + slots <= kScratchBytes;
+  a.share = shared ? fa::BwdShare::kShare : fa::BwdShare::kSameDq;
+  a.slots = shared ? ws + 2 * vec / sizeof(float) : nullptr;
   a.dq = dq;
   a.B = B;
   a.Hq = Hq;

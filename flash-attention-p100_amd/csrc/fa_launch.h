@@ -105,10 +105,12 @@ struct BwdPlan {
   int parts;   // (apart) workgroups that share one key tile's phase 1
   bool w4;     // width 64: the two-workgroups-per-CU shape
 };
-// has_w4: the launch has such an instantiation; slots: it has bwd_workspace_bytes'
-// slots (NK == N), so that parts may be more than one.
+// has_w4: the launch has such an instantiation. kShare: it has bwd_workspace_bytes'
+// slots (NK == N), so that parts may be more than one; kSameDq: it has not, but its
+// workgroups are those of the plan that shares, so that dQ is the same bit for bit.
+enum class BwdShare { kShare, kNone, kSameDq };
 BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, int window,
-                 bool has_w4, bool slots);
+                 bool has_w4, BwdShare share);
 // The most parts bwd_plan takes for a shape, whatever the call's options.
 int bwd_max_parts(int B, int Hq, int Hkv, int N, int D);
 struct BwdWorkspace {
@@ -168,7 +170,7 @@ struct BwdArgs {
   // Workspace: partial dK/dV of shared key tiles. Null: every key tile's phase
   // 1 stays in its own workgroup. Null counters turn the causal split off.
   float* slots = nullptr;
-  bool shared = false;  // the slots suffice for the parts of bwd_plan
+  BwdShare share = BwdShare::kSameDq;  // kShare: the slots suffice for bwd_plan's parts
   int dtype = kFP16;             // of q, k, v, dO, o, dk, dv and dq16
   const int* kv_len = nullptr;   // as FwdArgs::kv_len
   int window = 0;                // as FwdArgs::window
@@ -241,7 +243,7 @@ hipError_t launch_bwd_main_w(const BwdArgs& a);
 inline BwdPlan bwd_plan(const BwdArgs& a) {
   if (a.mask || a.block_rows) return {false, 1, false};
   const bool w4 = padded_head_dim(a.D) == 64 && !a.drop && !a.bias;
-  return bwd_plan(a.B, a.Hq, a.Hkv, a.N, key_rows(a.N, a.Nkv), a.D, a.causal, a.window, w4, a.shared);
+  return bwd_plan(a.B, a.Hq, a.Hkv, a.N, key_rows(a.N, a.Nkv), a.D, a.causal, a.window, w4, a.share);
 }
 hipError_t launch_fwd(const FwdArgs& a, const FwdPlan& plan, void* workspace);
 hipError_t launch_bwd_preprocess(const BwdArgs& a);

@@ -135,7 +135,7 @@ struct BwdCost {
 }  // namespace
 
 BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, int window,
-                 bool has_w4, bool slots) {
+                 bool has_w4, BwdShare share) {
   const BwdCost cost(B, Hq, Hkv, N, NK, D, causal, window);
   // One item per tile, two workgroups per CU where the grid fills both.
   const BwdPlan plain{false, 1,
@@ -162,9 +162,9 @@ BwdPlan bwd_plan(int B, int Hq, int Hkv, int N, int NK, int D, bool causal, int 
       consider({true, parts, w4}, cost.apart(parts, w4));
     }
   };
-  search(false, true);
-  if (has_w4) search(true, true);
-  if (!slots && best.parts > 1) {  // (the same workgroups, so that dQ is the same)
+  search(false, share != BwdShare::kNone);
+  if (has_w4) search(true, share != BwdShare::kNone);
+  if (share == BwdShare::kSameDq && best.parts > 1) {
     least = HUGE_VAL;
     search(best.w4, false);
   }
@@ -176,7 +176,7 @@ int bwd_max_parts(int B, int Hq, int Hkv, int N, int D) {
   for (const bool causal : {false, true})
     for (const bool w4 : {false, true}) {
       if (w4 && padded_head_dim(D) != 64) continue;
-      const BwdPlan p = bwd_plan(B, Hq, Hkv, N, N, D, causal, 0, w4, true);
+      const BwdPlan p = bwd_plan(B, Hq, Hkv, N, N, D, causal, 0, w4, BwdShare::kShare);
       if (p.parts > most) most = p.parts;
     }
   return most;

@@ -120,8 +120,8 @@ int fa_fwd_bnhd(const void* q, const void* k, const void* v, void* o, float* lse
  * among up to 24 workgroups, one for each of them (the most over causal and
  * dense calls of the shape: up to about 110 MB in all). Each part is rounded up to 256
  * bytes. 0 for an invalid shape. A workspace that ends after the pairs' slots is
- * taken too: key tiles are then not shared, which is slower on small grids, dq
- * is the same and dk, dv may differ in the last bits.
+ * taken too: key tiles are then not shared, which is slower on small grids, and
+ * results may differ in the last bits.
  */
 size_t fa_bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D);
 

