@@ -265,16 +265,15 @@ FwdPlan fwd_plan(const FwdArgs& a, bool workspace) {
     const double hi = a.causal ? fmax(1, fmin(NK, i1 + kofs)) : NK;
     return a.window > 0 ? fmin(hi, rows + a.window) : hi;
   };
-  double least, one_tile;  // (one_tile: workgroups of one 64-row tile)
+  double least, wgs;  // fa_fwd.hip's time and workgroups
   {  // fa_fwd.hip
     const double n = ceil_div(a.N, 64), stage = W > 128 ? 64 : 128;
     const bool pairs = a.causal && n > 1;
-    const double wgs = (pairs ? ceil_div(n, 2) : n) * BH;
+    wgs = (pairs ? ceil_div(n, 2) : n) * BH;
     const double first = ceil_div(keys(64, 64), stage), last = ceil_div(keys(64, 64 * n), stage);
     const double steps = 0.5 * (first + last) * n * BH / wgs, tiles = pairs ? 2 : 1;
     const FwdTimes& t = kTilesTimes[wi];
     const bool masked = a.N % 64 || a.kv_len || a.window > 0 || a.alibi || a.seg_start || NK != a.N;
-    one_tile = a.causal ? HUGE_VAL : wgs;
     least = 1 + (kTilesW4[wi] > 0 && wgs >= 2 * kCUs && !(a.causal && masked)
                      ? wgs / (2 * kCUs) * (steps * kTilesW4[wi] + tiles * t.ends)
                      : equal_time(t, wgs, steps, tiles));
@@ -291,11 +290,21 @@ FwdPlan fwd_plan(const FwdArgs& a, bool workspace) {
   // D=96, 14.7 against 17.9 at B=2 H=4 N=400 D=128 with one, 17.0 against 20.4 at
   // B=4 H=4 N=260 D=256 without. Of 1400 random calls with a bias 99 ran more than
   // 5% slower than on fa_fwd.hip without this rule, 4 with it.
+  // On causal grids of as few workgroups the estimates' errors decide, so another
+  // kernel is taken for a clear gain only: at most half a workgroup per CU, 7%, and
+  // with ALiBi, which costs fa_rows.hip more, 10% on up to one (14.1 us against 16.1
+  // at B=1 H=1 N=896 D=64): of 1400 random calls 46 without per-score inputs and 29
+  // with ALiBi were more than 5% slower than on fa_fwd.hip before, 35 and 3 now.
+  // (Not at width 256, where fa_fwd.hip's estimate errs the other way: 88 us
+  // there and 63 on fa_rows.hip at B=3 H=2 N=1727.)
+  const bool square = NK == a.N && !a.seg_start && a.window == 0;
   const double few = a.bias && W <= 64 ? kCUs / 2 : kCUs;
-  if (one_tile <= few && NK == a.N && !a.seg_start)
+  if (square && !a.causal && wgs <= few)
     least *= a.bias ? (W <= 64 ? 1.0 : W <= 96 ? 0.9 : 0.8) : (W <= 96 ? 1.0 : W <= 128 ? 0.85 : 0.8);
   else if (a.bias)
     least *= 1.6;
+  else if (square && a.causal && W <= 128)
+    least *= a.alibi && wgs <= kCUs ? 0.9 : wgs <= kCUs / 2 ? 0.93 : 1.0;
   if (a.drop && a.N % 128 == 0) least *= 0.85;
   // A launch's work-items and the row blocks' indices stay within 32 bits.
   constexpr double kMostItems = 4294967295.0;
