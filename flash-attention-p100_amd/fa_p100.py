@@ -52,15 +52,17 @@ _ext = _load_ext()
 # Rows and keys per block of a block-sparse layout (flash_attn's block_mask).
 BLOCK_SIZE = 128
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+# (bound once: _watched runs in every call, and the lookups took as long as the checks)
+_is_compiling, _is_tracing = torch.compiler.is_compiling, torch._C._is_tracing
+_functorch_level = torch._C._functorch.peek_interpreter_stack
 
 
 def _watched():
     """Whether a compiler, a tracer, a dispatch mode or a functorch transform sees
     this call as torch operators and Functions: the binding's entries are neither,
     and a graph recorded over them would hold empty tensors."""
-    return (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
-            or is_in_torch_dispatch_mode()
-            or torch._C._functorch.peek_interpreter_stack() is not None)
+    return (_is_compiling() or _is_tracing() or is_in_torch_dispatch_mode()
+            or _functorch_level() is not None)
 
 
 def _bnhd_storage(t):
